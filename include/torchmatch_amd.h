@@ -219,8 +219,9 @@ enum {
 };
 
 /* Device workspace the Sinkhorn calls below need.  The size depends on the
- * step form chosen for the shape (TORCHMATCH_AMD_SINKHORN_FUSED); keep that
- * variable unchanged between this query and the calls that use the
+ * form chosen for the shape (TORCHMATCH_AMD_SINKHORN_FUSED names a streaming
+ * step, TORCHMATCH_AMD_SINKHORN_RESIDENT=0 switches the resident solve off); keep
+ * those variables unchanged between this query and the calls that use the
  * workspace (a smaller workspace is refused with TM_ERR_WORKSPACE). */
 size_t tm_sinkhorn_workspace_bytes(int64_t B, int64_t N, int64_t M);
 
@@ -259,9 +260,11 @@ int tm_sinkhorn_read_stats(const void *workspace, int64_t B, int64_t N, int64_t 
  *   log_plan   device (B, N, M) output, may be NULL to skip the plan
  *   log_u, log_v  device (B, N), (B, M) outputs: the final scaling
  *              potentials (f = -eps * log_u, g = -eps * log_v)
- * With B >= 2 the steps of part of the batch run on a side stream of the
- * library's own (created on the first such call per device of `stream`,
- * default priority), forked from and joined back into `stream` with events:
+ * Matrices that fit the chip's registers are solved in one launch (cooperative
+ * when several workgroups share a problem; a `stream` under graph capture takes
+ * the streaming steps).  Otherwise, with B >= 2, the steps of part of the batch
+ * run on a side stream of the library's own (created on the first such call per
+ * device of `stream`, default priority), forked and joined with events:
  * the call stays stream-ordered on `stream`.  TORCHMATCH_AMD_SINKHORN_GROUPS=1
  * keeps every launch on `stream`, and so does a `stream` under graph capture.
  * Threading: calls from several host threads, on the same or different

@@ -1,0 +1,139 @@
+"""The resident Sinkhorn solve (csrc/sk_resident_kernel.h): the whole iteration
+in one launch.  Sizes at the edges of its tiles, one workgroup per problem and
+several (merged by every workgroup, and by column owners), steps it refuses
+and redoes from the cost, degenerate marginals, and a schedule longer than a
+launch takes (which the streaming steps serve).
+
+The oracle is run in float64.  A log-plan entry is one float32 rounding of a
+value up to 2^7 (4e-6) plus the potentials' error; every quantity is held to
+the 1e-5 the parity tests use.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import torchmatch_amd  # noqa: F401
+from oracle import sinkhorn as sk
+import sk_parity
+import workloads
+from torchmatch_amd.transport.matrix import Backend, solve
+
+pytestmark = pytest.mark.gpu
+
+# (B, N, M): one row, one column, tile edges and remainders of each layout
+SHAPES = [
+    (3, 1, 1), (2, 1, 70), (2, 70, 1), (2, 33, 64), (2, 64, 65), (3, 127, 96), (2, 130, 128),
+    (1, 260, 129), (2, 97, 193), (1, 500, 256), (2, 65, 257), (1, 129, 385), (1, 300, 513),
+    (1, 70, 769), (2, 40, 1024), (1, 130, 1025), (1, 34, 1537), (1, 150, 2048), (1, 20, 2049),
+    (1, 70, 4096), (300, 20, 24),
+]
+
+
+def _check(label, cost, a, b, eps, n_iter, device, rho=None, scaling=None, mask=None):
+    c = cost if mask is None else cost.masked_fill(~mask, float("inf"))
+    dev = {"a": a.to(device), "b": b.to(device), "reg": eps, "n_iter": n_iter,
+           "scaling": scaling, "mask": None if mask is None else mask.to(device)}
+    if rho is None:
+        ref = dict(zip(("plan", "f", "g"), sk.log_sinkhorn_plan(
+            c, eps=eps, n_iter=n_iter, a=a, b=b, scaling=scaling, dtype=torch.float64)))
+        got = dict(zip(("plan", "f", "g"), solve(cost.to(device), unpack=True, **dev)))
+    else:
+        ref = {"plan": sk.unbalanced_sinkhorn_plan(
+            c, eps=eps, n_iter=n_iter, rho=rho, a=a, b=b, scaling=scaling,
+            dtype=torch.float64)[0]}
+        got = {"plan": solve(cost.to(device), backend=Backend.UNBALANCED_SINKHORN, rho=rho,
+                             **dev)}
+    torch.cuda.synchronize()
+    for name, x in got.items():
+        err = sk_parity.logp_err(x, ref[name])
+        print(f"{label} {name}: {err:.2e}", flush=True)
+        assert err <= sk_parity.ELEM_BOUND, (label, name, err)
+
+
+@pytest.mark.parametrize("mode", [None, "exact"])
+@pytest.mark.parametrize("rho", [None, 0.7])
+def test_tile_edges(mode, rho, device, monkeypatch):
+    """Every step from P, and (``exact``) every step from the cost."""
+    if mode:
+        monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_RESIDENT", mode)
+    for B, N, M in SHAPES:
+        cost = workloads.sinkhorn_points(B, N, M, 8, seed=N + M)
+        if N > 4 and M > 8:
+            cost[0, 2, :] = float("inf")      # an empty row and column
+            cost[B - 1, :, 5] = float("inf")
+        _check(f"{(B, N, M)} rho {rho} {mode}", cost, workloads.dirichlet(B, N, seed=1),
+               workloads.dirichlet(B, M, seed=2), 0.05, 12, device, rho=rho)
+
+
+@pytest.mark.parametrize(("B", "N", "M"), [(2, 60, 90), (2, 700, 300), (1, 400, 1200)])
+def test_masked_and_scaled(B, N, M, device):
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=N)
+    mask = torch.rand(B, N, M, generator=torch.Generator().manual_seed(3)) < 0.7
+    a, b = workloads.dirichlet(B, N, seed=4), workloads.dirichlet(B, M, seed=5)
+    _check("scaled", cost, a, b, 0.03, 40, device, scaling=0.8, mask=mask)
+    # 200 epsilons: more runs than one launch takes
+    _check("long schedule", cost, a, b, 0.03, 200, device, scaling=0.985, mask=mask)
+
+
+@pytest.mark.parametrize(("B", "N", "M"), [(2, 60, 90), (2, 500, 300), (1, 300, 1200)])
+def test_degenerate_marginals(B, N, M, device):
+    """Zero and tiny masses, rows whose only partners carry none, and an epsilon
+    at which the row-maximum start underflows (the step is refused and redone)."""
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=M)
+    a, b = workloads.dirichlet(B, N, seed=6), workloads.dirichlet(B, M, seed=7)
+    a[:, 3] = 0.0
+    b[:, 4:9] = 0.0
+    a[:, 5] = 1e-30
+    b[0, 11] = 1e-25
+    cost[0, 7, :] = float("inf")
+    cost[0, 7, 4:9] = 0.25                    # allowed only where b is zero
+    _check("degenerate", cost, a, b, 0.05, 20, device)
+    _check("degenerate, unbalanced", cost, a, b, 0.05, 20, device, rho=0.3)
+    # |C| / eps up to 2000: float32 itself resolves the log plan to 1e-4 there,
+    # so the potentials (in units of the cost) are what is compared
+    args = {"reg": 5e-4, "n_iter": 15, "a": a.to(device), "b": b.to(device)}
+    ref = sk.log_sinkhorn_plan(cost, eps=5e-4, n_iter=15, a=a, b=b, dtype=torch.float64)
+    got = solve(cost.to(device), unpack=True, **args)
+    for x, r in zip(got[1:], ref[1:]):
+        # the float32 step epsilon of the solve: 3e-8 of potentials below 2
+        assert sk_parity.pot_err(x, r) <= 1e-6
+
+
+@pytest.mark.parametrize(("B", "N", "M", "rho"), [
+    (2, 1, 3, None), (2, 65, 64, 0.5), (3, 120, 250, None), (1, 300, 513, None),
+    (1, 260, 1000, 0.5),
+])
+def test_float64(B, N, M, rho, device):
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=N + 1).double()
+    a = workloads.dirichlet(B, N, seed=8).double()
+    b = workloads.dirichlet(B, M, seed=9).double()
+    if rho is None:
+        ref = sk.log_sinkhorn_plan(cost, eps=0.05, n_iter=40, a=a, b=b, dtype=torch.float64)[0]
+        got = solve(cost.to(device), a=a.to(device), b=b.to(device), reg=0.05, n_iter=40)
+    else:
+        ref = sk.unbalanced_sinkhorn_plan(cost, eps=0.05, n_iter=40, rho=rho, a=a, b=b,
+                                          dtype=torch.float64)[0]
+        got = solve(cost.to(device), backend=Backend.UNBALANCED_SINKHORN, rho=rho,
+                    a=a.to(device), b=b.to(device), reg=0.05, n_iter=40)
+    # values below 2^6, ulp 7e-15, a few roundings a step that do not add up
+    assert sk_parity.logp_err(got, ref) <= 2e-13
+
+
+@pytest.mark.parametrize(("B", "N", "M"), [(5, 120, 1028), (2, 300, 200)])
+def test_streaming_groups_same_bits(B, N, M, device, monkeypatch):
+    """The streaming step (which serves captures and matrices too large for the
+    chip) on shapes the resident solve takes by default: every batch-group
+    split gives the same bits, within the bound of the resident plan."""
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=31).to(device)
+    args = {"a": workloads.dirichlet(B, N, seed=1).to(device),
+            "b": workloads.dirichlet(B, M, seed=2).to(device), "reg": 0.05, "n_iter": 30}
+    resident = solve(cost, **args)
+    monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_FUSED", "1")
+    plans = []
+    for groups in ("1", "2", "4"):
+        monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_GROUPS", groups)
+        plans.append(solve(cost, **args))
+    assert torch.equal(plans[0], plans[1]) and torch.equal(plans[0], plans[2])
+    assert sk_parity.logp_err(plans[0], resident.cpu()) <= sk_parity.ELEM_BOUND

@@ -22,6 +22,7 @@ import shlex
 import subprocess
 import sys
 import sysconfig
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -33,7 +34,9 @@ OPS_SO = PKG / "_C.so"
 PROBE_SRC = PKG.parent / "bench_probes.hip"
 PROBE_SO = PKG.parent / "bench_probes.so"
 
-HIP_SOURCES = ["jv_batch.hip", "jv_large.hip", "jv_unpack.hip", "sinkhorn.hip", "sinkhorn64.hip"]
+HIP_SOURCES = ["jv_batch.hip", "jv_large.hip", "jv_unpack.hip", "sinkhorn.hip", "sinkhorn64.hip",
+               "sinkhorn_resident.hip", "sk_tiles_narrow.hip", "sk_tiles_wide.hip",
+               "sk_tiles_f64.hip"]
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = "gfx950"
 
@@ -65,12 +68,15 @@ def _run(cmd: list[str], verbose: bool) -> None:
 def build_cabi(verbose: bool = True) -> Path:
     """Compile the HIP kernels + C ABI into lib/libtorchmatch_amd.so."""
     LIB_DIR.mkdir(exist_ok=True)
-    objs = []
-    for src in HIP_SOURCES:
+
+    def compile_one(src: str) -> str:
         obj = LIB_DIR / (Path(src).stem + ".o")
         _run(["hipcc", *HIPCC_FLAGS, "-I", str(INCLUDE), "-c", str(CSRC / src), "-o", str(obj)],
              verbose)
-        objs.append(str(obj))
+        return str(obj)
+
+    with ThreadPoolExecutor(max_workers=4) as pool:
+        objs = list(pool.map(compile_one, HIP_SOURCES))
     tmp = CABI_SO.with_suffix(".so.tmp")
     _run(["hipcc", f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *objs,
           f"-Wl,-rpath,{ROCM / 'lib'}"], verbose)

@@ -55,6 +55,8 @@
 #include <mutex>
 
 #include "jv_batch.h"
+#include "sk_math.h"
+#include "sk_resident.h"
 #include "wave.h"
 
 namespace tmamd {
@@ -168,6 +170,10 @@ struct SinkhornLayout {
     size_t off_lu64, off_lv64, off_mu64, off_nu64, off_lu2, off_lv2;
     // per-column weights 2^(lv2 rounding residual), float32, B*M
     size_t off_lvw;
+    // the whole iteration in one launch from registers (sinkhorn_resident.hip)
+    // and its exchange buffer; the step forms above serve what it does not
+    SkResidentPlan res;
+    size_t off_xch;
 };
 
 __host__ __device__ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -256,6 +262,12 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
     L.n_chunk = (int)chunks;
     L.rows_per_chunk = (int)((N + chunks - 1) / chunks);
     choose_fused(L);
+    // the variables that name a step form ask for that form
+    L.res = SkResidentPlan{-1, 1, 0, 0, 1, 0};
+    if (getenv("TORCHMATCH_AMD_SINKHORN_FUSED") == nullptr &&
+        getenv("TORCHMATCH_AMD_SINKHORN_SHIFT_WINDOW") == nullptr)
+        L.res = sk_resident_plan(B, N, M, false);
+    const bool state64 = L.fused != kFzNone || L.res.cfg >= 0;
     size_t off = 0;
     L.off_k = off;
     off = align_up(off + sizeof(float) * (size_t)(B * N * M), 256);
@@ -278,16 +290,16 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
     if (L.fused)
         off = align_up(off + sizeof(float) * (size_t)(B * N), 256);
     L.off_lu64 = off;
-    if (L.fused)
+    if (state64)
         off = align_up(off + sizeof(double) * (size_t)(B * N), 256);
     L.off_lv64 = off;
-    if (L.fused)
+    if (state64)
         off = align_up(off + sizeof(double) * (size_t)(B * M), 256);
     L.off_mu64 = off;
-    if (L.fused)
+    if (state64)
         off = align_up(off + sizeof(double) * (size_t)(B * N), 256);
     L.off_nu64 = off;
-    if (L.fused)
+    if (state64)
         off = align_up(off + sizeof(double) * (size_t)(B * M), 256);
     L.off_lu2 = off;
     if (L.fused)
@@ -300,6 +312,8 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
         off = align_up(off + sizeof(float) * (size_t)(B * M), 256);
     L.off_stats = off;
     off += 256;
+    L.off_xch = off;
+    off = align_up(off + L.res.xch_bytes, 256);
     L.total = off;
     return L;
 }
@@ -905,51 +919,10 @@ __device__ __forceinline__ Lse fold_partial(float m, float s) {
     return Lse{s != 0.f ? m : -f_inf(), m == f_inf() ? f_inf() : s};
 }
 
-// Natural units per base-2 unit and back, float64: the fused step's K holds
-// -C'*log2(e)/e (k_of with s2 = -kLog2eD/e) and its potentials enter the
-// element loops scaled by kLog2eD, so 2^(K + p2) = e^(-C'/e + p) up to the
-// float32 roundings of K and p2, with no constant's rounding in the exponent.
-constexpr double kLog2eD = 1.4426950408889634074;
-constexpr double kLn2D = 0.69314718055994530942;
-
-// log2 of a float32 s > 0 in float64: s = m * 2^e with m in [sqrt(1/2),
-// sqrt(2)), e exact and the native log on m only.  The native log is
-// accurate near 1 but its error grows with |log2 s| (up to one float32 ulp
-// of the result, biased low), and a bias common to every row or column is
-// what the balanced potentials' neutral mode accumulates step after step.
-// +inf, 0 and NaN go to the native log directly.
-__device__ __forceinline__ double log2_split(float s) {
-    if (!(s > 0.f) || !__builtin_isfinite(s))
-        return (double)__builtin_amdgcn_logf(s);
-    int e = __builtin_amdgcn_frexp_expf(s);
-    float m = __builtin_amdgcn_frexp_mantf(s);  // [0.5, 1)
-    if (m < 0.70710678f) {
-        m *= 2.f;
-        e -= 1;
-    }
-    return (double)e + (double)__builtin_amdgcn_logf(m);
-}
-
-// log2 of a float64 sum s > 0: log2_split of its float32 rounding plus the
-// first-order term of the rounding (relative <= 2^-24, so the second-order
-// term is below 2^-49).
-__device__ __forceinline__ double log2_of_sum(double s) {
-    const float h = (float)s;
-    const float r = (float)(s - (double)h);  // exact: |r| <= ulp(h) / 2
-    return log2_split(h) + (double)(r * __builtin_amdgcn_rcpf(h) * kLog2e);
-}
-
-// 2^t of a float64 t as a float32, to about 1e-7 relative: 2^round(t)
-// exactly (ldexp) times the native 2^f of the float32 fraction f, |f| <= 1/2,
-// with f's own rounding r restored to first order (2^(f + r) = 2^f (1 + r ln 2)).
-__device__ __forceinline__ float pow2_of(double t) {
-    const double ti = fmin(fmax(rint(t), -300.0), 300.0);
-    const double fd = t - ti;
-    const float f = (float)fd;
-    const float r = (float)(fd - (double)f);
-    const float e = __builtin_amdgcn_exp2f(f);
-    return ldexpf(fmaf(e, r * kLn2, e), (int)ti);
-}
+// The fused step's K holds -C'*log2(e)/e (k_of with s2 = -kLog2eD/e) and its
+// potentials enter the element loops scaled by kLog2eD, so 2^(K + p2) =
+// e^(-C'/e + p) up to the float32 roundings of K and p2, with no constant's
+// rounding in the exponent.
 
 // A potential p (float64) enters the float32 element loops as p2 = fl(p *
 // log2 e) and the weight w = 2^(p * log2 e - p2) = 1 + (p*log2 e - p2) ln 2
@@ -1901,6 +1874,27 @@ int fused_groups(const SinkhornLayout &L) {
     return (int)(g < L.B ? g : L.B);
 }
 
+// The plan from the float64 potentials.
+int launch_plan64(const SinkhornLayout &L, const FusedPtrs &P, const float *cost,
+                  const uint8_t *keep, float e_final, float *log_plan, hipStream_t stream) {
+    const int64_t nK = L.B * L.N * L.M;
+    const int pvec = (L.M % 4) == 0 && ((uintptr_t)cost % 16) == 0 &&
+                     ((uintptr_t)keep % 4) == 0 && ((uintptr_t)log_plan % 16) == 0;
+    const dim3 pgrid(grid_for(pvec ? nK / 4 : nK, kMapBlock, 8192));
+    if (keep != nullptr)
+        TM_LAUNCH(sk_plan64<true>, pgrid, dim3(kMapBlock), 0, stream, cost, keep, P.lu64, P.lv64,
+                  log_plan, L.B, L.N, L.M, e_final, pvec);
+    else
+        TM_LAUNCH(sk_plan64<false>, pgrid, dim3(kMapBlock), 0, stream, cost, keep, P.lu64, P.lv64,
+                  log_plan, L.B, L.N, L.M, e_final, pvec);
+    return TM_OK;
+}
+
+// Not under capture: a cooperative launch cannot be recorded.
+bool resident_ok(const SinkhornLayout &L, const void *workspace, hipStream_t stream) {
+    return L.res.cfg >= 0 && ((uintptr_t)workspace % 16) == 0 && !stream_capturing(stream);
+}
+
 } // namespace
 
 extern "C" int tm_sinkhorn_prepare_f32(const float *cost, const uint8_t *keep, const float *a,
@@ -1932,8 +1926,12 @@ extern "C" int tm_sinkhorn_prepare_f32(const float *cost, const uint8_t *keep, c
     const int64_t n_flags = B * N > B * M ? B * N : B * M;
     TM_LAUNCH(sk_reset_flags, dim3(grid_for(n_flags, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
               stream, inf_row, B * N, inf_col, B * M, stats);
-    double *mu64 = L.fused ? reinterpret_cast<double *>(ws + L.off_mu64) : nullptr;
-    double *nu64 = L.fused ? reinterpret_cast<double *>(ws + L.off_nu64) : nullptr;
+    const bool resident = resident_ok(L, workspace, stream);
+    const bool state64 = L.fused != kFzNone || L.res.cfg >= 0;
+    double *mu64 = state64 ? reinterpret_cast<double *>(ws + L.off_mu64) : nullptr;
+    double *nu64 = state64 ? reinterpret_cast<double *>(ws + L.off_nu64) : nullptr;
+    if (resident)
+        k_eps = 0.f;  // the resident solve reads the cost, not K
     TM_LAUNCH(sk_log_marginal, dim3(grid_for(B * N, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
               stream, a, log_mu, mu64, B * N, stats, kFlagANeg);
     TM_LAUNCH(sk_log_marginal, dim3(grid_for(B * M, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
@@ -2039,6 +2037,22 @@ extern "C" int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, i
     const int64_t nK = B * N * M;
     const bool vec = (M % 4) == 0 && ((uintptr_t)log_v % 16) == 0;
     const bool fused = fused_ok(L, workspace);
+
+    if (resident_ok(L, workspace, stream)) {
+        const FusedPtrs P = fused_ptrs(L, ws, log_u, log_v, 0);
+        const SkResidentIo io{cost, keep, P.mu64, P.nu64, log_u, log_v, P.lu64, P.lv64,
+                              ws + L.off_xch};
+        const int rc = sk_resident_launch(L.res, io, B, N, M, eps_sched, n_iter, rho, false, stream);
+        if (rc == TM_OK)
+            return log_plan == nullptr
+                       ? TM_OK
+                       : launch_plan64(L, P, cost, keep, (float)eps_sched[n_iter - 1], log_plan,
+                                       stream);
+        if (rc != TM_ERR_UNSUPPORTED_SHAPE)
+            return rc;
+    }
+    if (L.res.cfg >= 0)
+        k_eps = 0.f;  // the preparation pass left K to this call
 
     TM_LAUNCH(sk_fill, dim3(grid_for(B * N, kMapBlock, 1 << 30)), dim3(kMapBlock), 0, stream,
               log_u, B * N, 0.f);
@@ -2157,17 +2171,8 @@ extern "C" int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, i
                       unbalanced ? 1 : 0);
     }
     if (log_plan != nullptr && fused) {
-        const FusedPtrs P = fused_ptrs(L, ws, log_u, log_v, 0);
-        const float e_final = (float)eps_sched[n_iter - 1];
-        const int pvec = (M % 4) == 0 && ((uintptr_t)cost % 16) == 0 &&
-                         ((uintptr_t)keep % 4) == 0 && ((uintptr_t)log_plan % 16) == 0;
-        const dim3 pgrid(grid_for(pvec ? nK / 4 : nK, kMapBlock, 8192));
-        if (keep != nullptr)
-            TM_LAUNCH(sk_plan64<true>, pgrid, dim3(kMapBlock), 0, stream, cost, keep, P.lu64,
-                      P.lv64, log_plan, B, N, M, e_final, pvec);
-        else
-            TM_LAUNCH(sk_plan64<false>, pgrid, dim3(kMapBlock), 0, stream, cost, keep, P.lu64,
-                      P.lv64, log_plan, B, N, M, e_final, pvec);
+        return launch_plan64(L, fused_ptrs(L, ws, log_u, log_v, 0), cost, keep,
+                             (float)eps_sched[n_iter - 1], log_plan, stream);
     } else if (log_plan != nullptr) {
         if (vec && ((uintptr_t)log_plan % 16) == 0)
             TM_LAUNCH(sk_plan4, dim3(grid_for(nK / 4, kMapBlock, 8192)), dim3(kMapBlock), 0,

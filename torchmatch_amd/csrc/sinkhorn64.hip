@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include "../../include/torchmatch_amd.h"
+#include "sk_resident.h"
 
 namespace {
 
@@ -28,7 +29,8 @@ constexpr int kStrip = 64;         // columns per strip
 constexpr int kGroups = kThreads / kStrip;
 
 struct Layout64 {
-    size_t off_k, off_logmu, off_lognu, off_infrow, off_infcol, total;
+    size_t off_k, off_logmu, off_lognu, off_infrow, off_infcol, off_xch, total;
+    tmamd::SkResidentPlan res;  // the whole iteration in one launch, where it fits
 };
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
@@ -46,6 +48,9 @@ Layout64 layout64(int64_t B, int64_t N, int64_t M) {
     off = align256(off + (size_t)(B * N));
     L.off_infcol = off;
     off = align256(off + (size_t)(B * M));
+    L.res = tmamd::sk_resident_plan(B, N, M, true);
+    L.off_xch = off;
+    off = align256(off + L.res.xch_bytes);
     L.total = off;
     return L;
 }
@@ -226,6 +231,19 @@ __global__ void sk64_plan(const double *__restrict__ K, const double *__restrict
     }
 }
 
+// The same plan from the cost: K = -C / eps (IEEE division).
+__global__ void sk64_plan_cost(const double *__restrict__ c, const double *__restrict__ log_u,
+                               const double *__restrict__ log_v, double *__restrict__ plan,
+                               int64_t B, int64_t N, int64_t M, double eps) {
+    const int64_t n = B * N * M;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+         k += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t r = k / M;
+        const int64_t b = r / N, j = k - r * M;
+        plan[k] = (log_u[r] + -c[k] / eps) + log_v[b * M + j];
+    }
+}
+
 unsigned grid_for(int64_t n, int per, int64_t cap) {
     int64_t g = (n + per - 1) / per;
     if (g < 1)
@@ -286,6 +304,23 @@ extern "C" int tm_sinkhorn_f64(const double *cost, const double *a, const double
                 log_mu, B * N);
     TM64_LAUNCH(sk64_log_marginal, dim3(grid_for(B * M, 256, 1 << 16)), dim3(256), stream, b,
                 log_nu, B * M);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const bool capturing =
+        hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+    if (L.res.cfg >= 0 && !capturing && ((uintptr_t)workspace % 16) == 0) {
+        const tmamd::SkResidentIo io{cost,  nullptr, log_mu,  log_nu,         log_u,
+                                     log_v, nullptr, nullptr, ws + L.off_xch};
+        const int rc = tmamd::sk_resident_launch(L.res, io, B, N, M, eps_sched, n_iter, rho, true,
+                                                 stream);
+        if (rc == TM_OK) {
+            if (log_plan != nullptr)
+                TM64_LAUNCH(sk64_plan_cost, map_grid, dim3(256), stream, cost, log_u, log_v,
+                            log_plan, B, N, M, eps_sched[n_iter - 1]);
+            return TM_OK;
+        }
+        if (rc != TM_ERR_UNSUPPORTED_SHAPE)
+            return rc;
+    }
     TM64_LAUNCH(sk64_row_flags, dim3(grid_for(B * N, 1, 1 << 16)), dim3(kThreads), stream, cost,
                 inf_row, B * N, M);
     TM64_LAUNCH(sk64_col_flags, dim3(grid_for(B * M, 256, 1 << 16)), dim3(256), stream, cost,

@@ -1,0 +1,1254 @@
+// sk_resident_kernel.h -- the whole Sinkhorn iteration in one launch, with the
+// matrix held in registers (gfx950).  Included by the sk_tiles_*.hip files, which
+// instantiate the tile configurations.
+//
+// A solve that launches one or two kernels per step is bound by those
+// launches (about 5 us each, 10 us per step) whenever the matrix is small, and
+// by re-reading the matrix when it is not.  256 CUs hold 128 MiB of VGPRs, so
+// here a problem's matrix is loaded once into the registers of G workgroups
+// and every step runs from there.
+//
+// The step.  With reference potentials (rl_i, c_j) the workgroups hold
+//     P_ij = e^(K_ij - rl_i - c_j)         K = -C / eps
+// and the potentials as multipliers a_i = e^(log_u_i + rl_i), b_j =
+// e^(log_v_j + c_j), so that the two half-steps of the log-domain iteration
+// are two matrix-vector products and no exponential:
+//     LSE_j(K_ij + log_v_j) = rl_i + log S_i     S_i = sum_j P_ij b_j
+//     LSE_i(K_ij + log_u_i) = c_j  + log T_j     T_j = sum_i P_ij a_i
+// and, balanced, a_i = mu_i / S_i, b_j = nu_j / T_j.  P is rounded to float32
+// once (relative 2^-24 per entry; the K of the streaming step is rounded to
+// float32 at |K| ~ 40, about 2^-19), lane sums are float32 of TC or TR terms,
+// sums across lanes and waves and the multipliers are float64.  The float32
+// copies of a and b that the products read carry their rounding error over
+// to the next step's rounding (ea, eb), so that a fixed rounding of a
+// converged multiplier does not drive the potentials' neutral mode
+// (log_u + c, log_v - c) step after step.
+//
+// When that is exact enough.  P underflows below 2^-149 and its absolute error
+// there is below 2^-126 max(a, b) per entry; a step is accepted only while
+// every S_i and T_j lies in [2^-60, 2^60] and every multiplier is at most
+// 2^20, so what is lost is below 2^-32 of a sum.  A step outside the window
+// (and the first) is done exactly from the cost, with the maximum taken out
+// of every sum, the reference's logsumexp, and P is rebuilt around the new
+// potentials.  A row or column whose LSE is not finite keeps its potential, as
+// the reference's isfinite rule has it.  When epsilon changes, P is rebuilt
+// from the cost around the current potentials and the step goes on.
+//
+// Several workgroups per problem.  Each holds `rows` whole rows, so the row
+// half-step is local; the column sums are exchanged through global memory in
+// 64-bit words that carry 32 bits of payload and the number of the exchange,
+// written and polled with relaxed agent-scope atomics.  A word is its own
+// flag: no fence and no L2 write-back is needed, and double buffering by the
+// exchange's parity keeps a slot until every reader has moved on.  With few
+// columns every workgroup merges all of them (one hop, `direct`); else
+// workgroup g owns a range of columns, merges it and sends its multipliers to
+// the others (two hops).  Such a grid is launched cooperatively, which
+// guarantees that all its workgroups are resident, and every wait is bounded
+// in time.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+
+#include <utility>
+
+#include "sk_math.h"
+#include "sk_resident.h"
+#include "wave.h"
+
+namespace tmamd {
+namespace {
+
+constexpr double kSumLo = 0x1p-60, kSumHi = 0x1p60, kMulHi = 0x1p20;
+// a wait longer than this (100 MHz ticks) ends the solve with NaN potentials
+constexpr uint64_t kWaitTicks = 400000000ull;
+
+// The log unit of each type: base 2 on the native v_exp_f32 for float costs,
+// natural with the library's exp / log for double costs.
+template <typename T> struct Unit;
+template <> struct Unit<float> {
+    static constexpr int kPartWords = 1;
+    double s2;
+    __device__ explicit Unit(double eps) : s2(-kLog2eD / (double)(float)eps) {}
+    __device__ double kval(float c) const { return (double)c * s2; }
+    static __device__ float term(double t) { return __builtin_amdgcn_exp2f((float)t); }
+    static __device__ double logm(double s) { return log2(s); }
+    static __device__ double expm(double t) { return exp2(t); }
+    static __device__ double log_fast(double s) { return log2_of_sum(s); }
+    static __device__ double exp_fast(double t) { return (double)pow2_of(t); }
+    // 1 / s: one Newton step on the native reciprocal (about 2^-46)
+    static __device__ double recip(double s) {
+        const double r = __builtin_amdgcn_rcp(s);
+        return fma(fma(-s, r, 1.0), r, r);
+    }
+    static __device__ double of_nat(double x) { return x * kLog2eD; }
+    static __device__ double to_nat(double x) { return x * kLn2D; }
+    static __device__ double of_exp2(int e) { return (double)e; }
+    // P from its exponent, |error| about one ulp (NaN stays NaN)
+    static __device__ float build(double t) {
+        t = t < -300.0 ? -300.0 : t;
+        const double ti = rint(t);
+        return ldexpf(__builtin_amdgcn_exp2f((float)(t - ti)), (int)fmin(ti, 300.0));
+    }
+};
+template <> struct Unit<double> {
+    static constexpr int kPartWords = 2;
+    double eps;
+    __device__ explicit Unit(double e) : eps(e) {}
+    __device__ double kval(double c) const { return -c / eps; }
+    static __device__ double term(double t) { return exp(t); }
+    static __device__ double logm(double s) { return log(s); }
+    static __device__ double expm(double t) { return exp(t); }
+    static __device__ double log_fast(double s) { return log(s); }
+    static __device__ double exp_fast(double t) { return exp(t); }
+    static __device__ double recip(double s) { return 1.0 / s; }
+    static __device__ double of_nat(double x) { return x; }
+    static __device__ double to_nat(double x) { return x; }
+    static __device__ double of_exp2(int e) { return (double)e * kLn2D; }
+    static __device__ double build(double t) { return exp(t); }
+};
+
+__device__ __forceinline__ double shift_of(double m) { return isinf(m) ? 0.0 : m; }
+
+__device__ __forceinline__ double pack_d(uint32_t lo, uint32_t hi) {
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// a + b after exchanging the halves the lane does not keep: lanes of the
+// lower half (of 64, or of each 32) hold a's pair sum, the others b's
+__device__ __forceinline__ double pair_swap32(double a, double b) {
+    const uint64_t ua = (uint64_t)__double_as_longlong(a), ub = (uint64_t)__double_as_longlong(b);
+    const u32x2 lo = __builtin_amdgcn_permlane32_swap((uint32_t)ua, (uint32_t)ub, false, false);
+    const u32x2 hi = __builtin_amdgcn_permlane32_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32),
+                                                      false, false);
+    return pack_d(lo[0], hi[0]) + pack_d(lo[1], hi[1]);
+}
+__device__ __forceinline__ double pair_swap16(double a, double b) {
+    const uint64_t ua = (uint64_t)__double_as_longlong(a), ub = (uint64_t)__double_as_longlong(b);
+    const u32x2 lo = __builtin_amdgcn_permlane16_swap((uint32_t)ua, (uint32_t)ub, false, false);
+    const u32x2 hi = __builtin_amdgcn_permlane16_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32),
+                                                      false, false);
+    return pack_d(lo[0], hi[0]) + pack_d(lo[1], hi[1]);
+}
+__device__ __forceinline__ float pair_swap32(float a, float b) {
+    const u32x2 x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                     false);
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+__device__ __forceinline__ float pair_swap16(float a, float b) {
+    const u32x2 x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                     false);
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+template <int CTRL> __device__ __forceinline__ float dpp_t(float x) { return dpp_full_f<CTRL>(x); }
+template <int CTRL> __device__ __forceinline__ double dpp_t(double x) { return dpp_full_d<CTRL>(x); }
+
+constexpr int kDppRowRor4 = 0x124, kDppRowRor8 = 0x128;  // rotate within 16 lanes
+constexpr int kDppRowNewBcast0 = 0x150;                  // lane n of each 16 to all of them
+
+// Sums of four values over each 16 lanes: lanes with lane % 4 == i get value
+// i's.  Two halving steps in the value's type (each lane keeps half of the
+// values and sends the other half), the last two in float64.
+template <typename T>
+__device__ __forceinline__ double row16_sum4(const T (&s)[4], bool odd, bool odd2) {
+    const T y0 = (odd ? s[1] : s[0]) + dpp_t<kDppQuadXor1>(odd ? s[0] : s[1]);
+    const T y1 = (odd ? s[3] : s[2]) + dpp_t<kDppQuadXor1>(odd ? s[2] : s[3]);
+    const T z = (odd2 ? y1 : y0) + dpp_t<kDppQuadXor2>(odd2 ? y0 : y1);
+    double d = (double)z;
+    d += dpp_full_d<kDppRowRor8>(d);
+    d += dpp_full_d<kDppRowRor4>(d);
+    return d;
+}
+
+// f(0), f(1), ... f(N - 1) with the index as a constant expression
+template <typename Fn, int... I>
+__device__ __forceinline__ void unroll_seq(Fn &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename Fn> __device__ __forceinline__ void unroll(Fn &&f) {
+    unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ float readlane_t(float x, int lane) { return readlane_f(x, lane); }
+__device__ __forceinline__ double readlane_t(double x, int lane) { return readlane_d(x, lane); }
+
+__device__ __forceinline__ void put_word(uint64_t *p, uint32_t payload, uint32_t tag) {
+    __hip_atomic_store(p, ((uint64_t)tag << 32) | payload, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get_word(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A bounded wait: false once the launch has waited longer than kWaitTicks.
+struct Waiter {
+    uint32_t polls = 0;
+    uint64_t start = 0;
+    __device__ bool more() {
+        if ((++polls & 1023u) != 0)
+            return true;
+        const uint64_t now = wall_clock64();
+        if (start == 0)
+            start = now;
+        return now - start < kWaitTicks;
+    }
+};
+
+// Payload of the word at p once its tag is `tag` (bit 0 of the tag is the
+// sender's bad flag, OR-ed into `bad`).
+__device__ __forceinline__ uint32_t wait_word(const uint64_t *p, uint32_t tag, uint32_t &bad,
+                                              int &timed_out) {
+    uint64_t w = get_word(p);
+    Waiter wt;
+    while (((uint32_t)(w >> 32) | 1u) != (tag | 1u)) {
+        if (!wt.more()) {
+            timed_out = 1;
+            break;
+        }
+        w = get_word(p);
+    }
+    bad |= (uint32_t)(w >> 32) & 1u;
+    return (uint32_t)w;
+}
+
+// One workgroup's share of a problem, R rows of up to CW columns, in one of
+// two layouts of a wave (wr, wc) (WC waves side by side share RW rows):
+//   LC = 64  the lanes span the columns: lane l holds columns
+//            (k*WC + wc)*64 + l, k < TC, of RW = TR rows; for wide matrices
+//   LC = 16  four groups of 16 lanes: lane (h, c) holds columns
+//            (k*WC + wc)*16 + c of the rows 4*r + h, r < TR, so RW = 4*TR; for
+//            up to 256 columns per wave, where the other layout would spend
+//            more on reducing a row over 64 lanes than on its products
+template <typename T, int NW_, int LC_, int WC_, int TC_, int TR_, bool SOLO_> struct Cfg {
+    using Type = T;
+    static constexpr int NW = NW_, LC = LC_, WC = WC_, TC = TC_, TR = TR_;
+    static constexpr bool SOLO = SOLO_;                    // one workgroup per problem
+    static constexpr int NT = NW * 64;                     // threads
+    static constexpr int WR = NW / WC;
+    static constexpr int RW = LC == 64 ? TR : 4 * TR;      // rows of a wave
+    static constexpr int NV = RW / 4;                      // row sums per lane, see lane_row
+    static constexpr int R = WR * RW;
+    static constexpr int ETC = (LC * TC + 63) / 64;        // columns per lane, exact step
+    static constexpr int CW = WC * 64 * ETC;
+    static constexpr int NK = (CW + NT - 1) / NT;          // columns per thread
+    static constexpr int KC = SOLO ? NK : 1;               // owned columns per thread
+    static constexpr int PW = Unit<T>::kPartWords;  // words of a column partial
+    static constexpr int XW = PW + 1;               // words of an exact partial (max, sum)
+    static constexpr int BW = PW + 2;               // words of an exact broadcast (c, b)
+    static_assert(RW <= 64 && RW % 4 == 0, "one row per lane");
+    static __device__ __forceinline__ int col(int k, int wc, int lane) {
+        return (k * WC + wc) * LC + (lane & (LC - 1));
+    }
+};
+
+template <typename F> struct Shared {
+    using T = typename F::Type;
+    double c[F::CW];               // column references, all columns
+    double rs[F::WC * F::R];       // row sums of each column wave
+    double rl[F::R];               // row references (exact step: log_u)
+    double xs[F::NT];              // split column sums
+    double bd[F::KC * F::NT];        // owned columns: multiplier and marginal
+    double nu[F::KC * F::NT];        // (unbalanced: in log units)
+    T b[F::CW];
+    T cp[F::WR * F::CW];           // column sums of each row wave
+    float cm[F::WR * F::CW];       // exact step: their maxima
+    float rm[F::WC * F::R];        // exact step: row maxima
+    float eb[F::KC * F::NT];
+    uint8_t dead[F::KC * F::NT];
+    int flag_row[2], flag_all[2], abort;
+};
+#define TM_LDS __attribute__((address_space(3)))
+template <typename F> using SharedP = TM_LDS Shared<F> *;
+
+// The row a lane keeps, of its wave's RW: where the reductions leave the row
+// sums (lanes past RW keep none).
+__device__ __forceinline__ int lane_row(int lane) { return 4 * (lane & 15) + (lane >> 4); }
+
+struct Row {
+    double lmu, mu;   // marginal: log units, linear
+    double rl, a;     // reference, multiplier of the last accepted step
+    double lu;        // log_u where it is explicit (see `derived`)
+    float ea;         // rounding carried by the float32 copy of a
+    bool dead;        // the LSE is not finite: the potential keeps its value
+    bool derived;     // balanced: log_u is log(a) - rl
+};
+
+// What a workgroup works on: one problem's rows and exchange buffers.
+struct Job {
+    const void *C;
+    const uint8_t *keep;
+    const double *lnu;
+    uint64_t *part, *cast;
+    int M, Mp, G, g, nrow, j0, cn, direct, unbal;
+};
+
+template <typename F, typename T>
+__device__ __forceinline__ void load_rows(const Job &J, int row, int wc, int lane,
+                                          T (&c)[F::ETC]) {
+    const T *C = static_cast<const T *>(J.C);
+    const int64_t base = (int64_t)min(row, J.nrow - 1) * J.M;
+#pragma unroll
+    for (int k = 0; k < F::ETC; ++k) {
+        const int j = (k * F::WC + wc) * 64 + lane;
+        const int64_t o = base + min(j, J.M - 1);
+        bool ok = row < J.nrow && j < J.M;
+        if (J.keep != nullptr)
+            ok = ok && J.keep[o] != 0;
+        c[k] = ok ? C[o] : (T)INFINITY;
+    }
+}
+
+// One step from the cost, the maximum taken out of every sum (the reference's
+// logsumexp and its rules); sets the references and multipliers around the
+// new potentials.  Not inlined: it runs once per problem (and after a refused
+// step) and would cost the step loop its registers.
+template <typename F>
+__device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, double eps, double damp,
+                                        uint32_t seq) {
+    using T = typename F::Type;
+    using U = Unit<T>;
+    constexpr int WC = F::WC, WR = F::WR, TC = F::ETC, TR = F::RW, R = F::R, CW = F::CW;
+    constexpr int XW = F::XW, PW = F::PW, BW = F::BW;
+    constexpr int RG = TC <= 4 ? 4 : 2;  // rows in flight
+    const int t = (int)threadIdx.x, lane = lane_id();
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wr = wid / WC, wc = wid % WC;
+    const int M = J.M, Mp = J.Mp, G = J.G;
+    const U u(eps);
+    {
+        double lvk[TC];
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            const int j = (k * WC + wc) * 64 + lane;
+            lvk[k] = U::logm((double)S->b[j]) - S->c[j];
+        }
+#pragma unroll 1
+        for (int r0 = 0; r0 < TR; r0 += RG) {
+            T c[RG][TC];
+#pragma unroll
+            for (int r = 0; r < RG; ++r)
+                load_rows<F>(J, wr * TR + r0 + r, wc, lane, c[r]);
+#pragma unroll
+            for (int r = 0; r < RG; ++r) {
+                double x[TC];
+                float m = -INFINITY;
+#pragma unroll
+                for (int k = 0; k < TC; ++k) {
+                    x[k] = u.kval(c[r][k]) + lvk[k];
+                    m = fmaxf(m, (float)x[k]);
+                }
+                m = wave_max_all(m);
+                const double sh = shift_of(m);
+                double s = 0.0;
+#pragma unroll
+                for (int k = 0; k < TC; ++k)
+                    s += (double)U::term(x[k] - sh);
+                s = wave_sum_all_d(s);
+                if (lane == 0) {
+                    S->rm[wc * R + wr * TR + r0 + r] = m;
+                    S->rs[wc * R + wr * TR + r0 + r] = s;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    double lse = 0.0;
+    const int rho = lane_row(lane), row = wr * TR + rho;
+    const bool has = rho < TR && row < J.nrow;
+    if (has) {
+        float m = S->rm[row];
+#pragma unroll
+        for (int w = 1; w < WC; ++w)
+            m = fmaxf(m, S->rm[w * R + row]);
+        const double sh = shift_of(m);
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < WC; ++w) {
+            const double sw = S->rs[w * R + row];
+            if (sw != 0.0)
+                s += WC == 1 ? sw : sw * U::expm(shift_of(S->rm[w * R + row]) - sh);
+        }
+        lse = U::logm(s) + sh;
+        if (W.derived && !W.dead && !J.unbal)
+            W.lu = U::logm(W.a) - W.rl;
+        W.dead = !isfinite(lse);
+        if (!W.dead) {
+            const double d = W.lmu - lse;
+            W.lu = J.unbal ? damp * d : d;
+        }
+        W.derived = false;
+    }
+    if (wc == 0 && rho < TR)
+        S->rl[row] = has ? W.lu : -INFINITY;
+    __syncthreads();
+    {
+        float m[TC];
+        T s[TC];
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            m[k] = -INFINITY;
+            s[k] = (T)0;
+        }
+#pragma unroll 1
+        for (int r0 = 0; r0 < TR; r0 += RG) {
+            T c[RG][TC];
+#pragma unroll
+            for (int r = 0; r < RG; ++r)
+                load_rows<F>(J, wr * TR + r0 + r, wc, lane, c[r]);
+#pragma unroll
+            for (int r = 0; r < RG; ++r) {
+                const double l = S->rl[wr * TR + r0 + r];
+#pragma unroll
+                for (int k = 0; k < TC; ++k)
+                    m[k] = fmaxf(m[k], (float)(u.kval(c[r][k]) + l));
+            }
+        }
+#pragma unroll 1
+        for (int r0 = 0; r0 < TR; r0 += RG) {
+            T c[RG][TC];
+#pragma unroll
+            for (int r = 0; r < RG; ++r)
+                load_rows<F>(J, wr * TR + r0 + r, wc, lane, c[r]);
+#pragma unroll
+            for (int r = 0; r < RG; ++r) {
+                const double l = S->rl[wr * TR + r0 + r];
+#pragma unroll
+                for (int k = 0; k < TC; ++k)
+                    s[k] += U::term((u.kval(c[r][k]) + l) - shift_of(m[k]));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            const int j = (k * WC + wc) * 64 + lane;
+            S->cm[wr * CW + j] = m[k];
+            S->cp[wr * CW + j] = s[k];
+        }
+    }
+    __syncthreads();
+    const uint32_t tag = seq << 1;
+    uint64_t *pw = J.part + (size_t)(seq & 1) * G * XW * Mp;
+    uint64_t *cw = J.cast + (size_t)(seq & 1) * BW * Mp;
+    int late = 0;
+    uint32_t unused = 0;
+    // this workgroup's (max, sum) of column j
+    auto local_pair = [&](int j, float &m, double &s) {
+        m = S->cm[j];
+#pragma unroll
+        for (int w = 1; w < WR; ++w)
+            m = fmaxf(m, S->cm[w * CW + j]);
+        const double sh = shift_of(m);
+        s = 0.0;
+#pragma unroll 1
+        for (int w = 0; w < WR; ++w) {
+            const double sw = (double)S->cp[w * CW + j];
+            if (sw != 0.0)
+                s += sw * U::expm(shift_of(S->cm[w * CW + j]) - sh);
+        }
+    };
+    if (G > 1) {
+        for (int j = t; j < M; j += F::NT) {
+            float m;
+            double s;
+            local_pair(j, m, s);
+            uint64_t *p = pw + (size_t)J.g * XW * Mp + j;
+            put_word(p, __float_as_uint(m), tag);
+            if constexpr (PW == 1) {
+                put_word(p + Mp, __float_as_uint((float)s), tag);
+            } else {
+                const uint64_t q = (uint64_t)__double_as_longlong(s);
+                put_word(p + Mp, (uint32_t)q, tag);
+                put_word(p + 2 * (size_t)Mp, (uint32_t)(q >> 32), tag);
+            }
+        }
+    }
+#pragma unroll 1
+    for (int jl = t; jl < J.cn; jl += F::NT) {
+        const int j = J.j0 + jl;
+        float m = -INFINITY;
+        double s = 0.0;
+        if (G == 1) {
+            local_pair(j, m, s);
+        } else {
+            // running merge in workgroup order, the same in every workgroup
+            // that merges this column
+#pragma unroll 1
+            for (int q = 0; q < G; ++q) {
+                const uint64_t *p = pw + (size_t)q * XW * Mp + j;
+                const float mq = __uint_as_float(wait_word(p, tag, unused, late));
+                double sq;
+                const uint32_t lo = wait_word(p + Mp, tag, unused, late);
+                if constexpr (PW == 1)
+                    sq = (double)__uint_as_float(lo);
+                else
+                    sq = pack_d(lo, wait_word(p + 2 * (size_t)Mp, tag, unused, late));
+                const float mn = fmaxf(m, mq);
+                const double sh = shift_of(mn);
+                s = (s != 0.0 ? s * U::expm(shift_of(m) - sh) : 0.0) +
+                    (sq != 0.0 ? sq * U::expm(shift_of(mq) - sh) : 0.0);
+                m = mn;
+            }
+        }
+        const double l = U::logm(s) + shift_of(m);
+        double lv = U::logm(S->bd[jl]) - S->c[j];
+        const bool dc = !isfinite(l);
+        if (!dc) {
+            const double d = U::of_nat(J.lnu[j]) - l;
+            lv = J.unbal ? damp * d : d;
+        }
+        const double cr = !dc ? l : isfinite(lv) ? -lv : 0.0;
+        const double b = U::expm(lv + cr);
+        S->bd[jl] = b;
+        S->eb[jl] = 0.f;
+        S->dead[jl] = dc;
+        S->c[j] = cr;
+        S->b[j] = (T)b;
+        if (G > 1 && !J.direct) {
+            const uint64_t q = (uint64_t)__double_as_longlong(cr);
+            put_word(cw + j, (uint32_t)q, tag);
+            put_word(cw + Mp + j, (uint32_t)(q >> 32), tag);
+            if constexpr (PW == 1) {
+                put_word(cw + 2 * (size_t)Mp + j, __float_as_uint((float)b), tag);
+            } else {
+                const uint64_t qb = (uint64_t)__double_as_longlong(b);
+                put_word(cw + 2 * (size_t)Mp + j, (uint32_t)qb, tag);
+                put_word(cw + 3 * (size_t)Mp + j, (uint32_t)(qb >> 32), tag);
+            }
+        }
+    }
+    if (G > 1 && !J.direct) {
+        __syncthreads();
+        for (int j = t; j < M; j += F::NT) {
+            const uint32_t lo = wait_word(cw + j, tag, unused, late);
+            S->c[j] = pack_d(lo, wait_word(cw + Mp + j, tag, unused, late));
+            const uint32_t b0 = wait_word(cw + 2 * (size_t)Mp + j, tag, unused, late);
+            if constexpr (PW == 1)
+                S->b[j] = __uint_as_float(b0);
+            else
+                S->b[j] = pack_d(b0, wait_word(cw + 3 * (size_t)Mp + j, tag, unused, late));
+        }
+    }
+    if (late)
+        S->abort = 1;
+    if (has) {
+        W.rl = !W.dead ? lse : isfinite(W.lu) ? -W.lu : 0.0;
+        W.a = U::expm(W.lu + W.rl);
+        W.ea = 0.f;
+    }
+    __syncthreads();
+}
+
+// Epsilon changed: move the references by powers of two to the current
+// potentials (each multiplier back to [1, 2)).
+template <typename F>
+__device__ __noinline__ void recentre(SharedP<F> S, const Job &J, Row &W) {
+    using T = typename F::Type;
+    using U = Unit<T>;
+    for (int j = (int)threadIdx.x; j < J.M; j += F::NT) {
+        const double b = (double)S->b[j];
+        int e = 0;
+        if (b > 0.0 && isfinite(b))
+            e = ilogb(b);
+        S->b[j] = (T)ldexp(b, -e);
+        S->c[j] -= U::of_exp2(e);
+        const int jl = j - J.j0;
+        if (jl >= 0 && jl < J.cn)
+            S->bd[jl] = ldexp(S->bd[jl], -e);
+    }
+    // rows the lane does not have hold a = 0
+    if (W.a > 0.0 && isfinite(W.a)) {
+        const int e = ilogb(W.a);
+        W.a = ldexp(W.a, -e);
+        W.rl -= U::of_exp2(e);
+    }
+}
+
+// Start state of a problem: potentials 0, marginals in log units and linear.
+template <typename F>
+__device__ __noinline__ void start_problem(SharedP<F> S, const Job &J, Row &W, const double *lmu) {
+    using T = typename F::Type;
+    using U = Unit<T>;
+    const int t = (int)threadIdx.x;
+    W = Row{-INFINITY, 0.0, 0.0, 0.0, 0.0, 0.f, false, false};
+    const int rho = lane_row(lane_id()), row = (t >> 6) / F::WC * F::RW + rho;
+    if (rho < F::RW && row < J.nrow) {
+        W.lmu = U::of_nat(lmu[row]);
+        W.mu = U::expm(W.lmu);
+        W.a = 1.0;
+    }
+    for (int j = t; j < F::CW; j += F::NT) {
+        S->c[j] = j < J.M ? 0.0 : INFINITY;  // columns past M: P = 0, b = 0
+        S->b[j] = j < J.M ? (T)1 : (T)0;
+    }
+    for (int jl = t; jl < F::KC * F::NT; jl += F::NT) {
+        S->bd[jl] = 1.0;
+        S->eb[jl] = 0.f;
+        S->dead[jl] = 0;
+        const double l = jl < J.cn ? U::of_nat(J.lnu[J.j0 + jl]) : -INFINITY;
+        S->nu[jl] = J.unbal ? l : U::expm(l);
+    }
+    __syncthreads();
+}
+
+// The potentials of a finished problem (NaN when a wait ran out).
+template <typename F>
+__device__ __noinline__ void finish_problem(SharedP<F> S, const Job &J, Row &W,
+                                            typename F::Type *log_u, double *lu64,
+                                            typename F::Type *log_v, double *lv64) {
+    using T = typename F::Type;
+    using U = Unit<T>;
+    const int t = (int)threadIdx.x;
+    const bool failed = S->abort != 0;
+    const int rho = lane_row(lane_id()), row = (t >> 6) / F::WC * F::RW + rho;
+    if ((t >> 6) % F::WC == 0 && rho < F::RW && row < J.nrow) {
+        if (W.derived && !W.dead && !J.unbal)
+            W.lu = U::logm(W.a) - W.rl;
+        const double x = failed ? NAN : U::to_nat(W.lu);
+        log_u[row] = (T)x;
+        if (lu64 != nullptr)
+            lu64[row] = x;
+    }
+    if (!J.direct || J.g == 0) {
+        for (int jl = t; jl < J.cn; jl += F::NT) {
+            const double x =
+                failed ? NAN : U::to_nat(U::logm(S->bd[jl]) - S->c[J.j0 + jl]);
+            log_v[J.j0 + jl] = (T)x;
+            if (lv64 != nullptr)
+                lv64[J.j0 + jl] = x;
+        }
+    }
+    __syncthreads();  // the next problem rewrites the shared state
+}
+
+template <typename F>
+__global__ void __launch_bounds__(F::NT)
+sk_resident(const ResArgs A) {
+    using T = typename F::Type;
+    using U = Unit<T>;
+    constexpr int LC = F::LC, WC = F::WC, WR = F::WR, TC = F::TC, TR = F::TR, R = F::R;
+    constexpr int CW = F::CW, RW = F::RW, NV = F::NV, KC = F::KC, XW = F::XW, PW = F::PW;
+    constexpr int BW = F::BW;
+    constexpr bool SOLO = F::SOLO;
+    __shared__ Shared<F> S;
+    const SharedP<F> SP = (SharedP<F>)&S;
+
+    const int t = (int)threadIdx.x;
+    const int lane = lane_id();
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wr = wid / WC, wc = wid % WC;
+    const int G = SOLO ? 1 : A.G, M = A.M, Mp = A.Mp;
+    const bool direct = SOLO || A.direct;
+    const int g = SOLO ? 0 : (int)blockIdx.x % G;
+    const int cluster = SOLO ? (int)blockIdx.x : (int)blockIdx.x / G;
+    const bool unbal = A.rho > 0.0;
+    const int i0 = g * A.rows;
+    const int nrow = A.N - i0 < A.rows ? A.N - i0 : A.rows;
+    const int j0 = direct ? 0 : min(g * A.cpo, M);
+    const int cn = direct ? M : min(A.cpo, M - j0);
+    // column merge: cnp = 16, 32, ... threads span the owned columns, and when
+    // more than one such group fits the workgroup the groups share the G
+    // partials of each column (group sp takes q = sp, sp + split, ...), so
+    // that no load instruction goes out half empty: each costs about 16
+    // cycles of address processing whatever it fetches
+    int cnp = 16;
+    while (cnp < A.cpo && cnp < F::NT)
+        cnp *= 2;
+    const int split = SOLO ? 1 : F::NT / cnp;
+    const int per = (G + split - 1) / split;  // partials of a column per thread
+    uint64_t *part = A.xch + (size_t)cluster * 2 * ((size_t)G * XW + BW) * Mp;
+    uint64_t *cast = part + (size_t)2 * G * XW * Mp;
+    const int rho = lane_row(lane), lrow = wr * RW + rho;  // the lane's row
+    const bool has = rho < RW && lrow < nrow;
+    const bool odd = lane & 1, odd2 = lane & 2;
+    uint32_t seq = 0;
+    if (t == 0)
+        S.abort = 0;
+    __syncthreads();
+
+    for (int64_t prob = cluster; prob < A.B; prob += A.clusters) {
+        const int64_t off = (prob * A.N + i0) * (int64_t)M;
+        const Job J{static_cast<const T *>(A.cost) + off, A.keep ? A.keep + off : nullptr,
+                    A.lnu + prob * M, part, cast, M, Mp, G, g, nrow, j0, cn, direct, unbal};
+        Row W;
+        start_problem<F>(SP, J, W, A.lmu + prob * A.N + i0);
+
+        // What the next step starts from: `trial`, P around the row maxima and
+        // log_v = 0 (the first step; refused where columns underflow);
+        // `exact`, the cost; `moved`, P around the current potentials.
+        enum { kTrial, kExact, kMoved } start = A.exact_only ? kExact : kTrial;
+        int it = 0, seg = 0;
+        while (it < A.n_iter && !S.abort) {
+            if (start == kExact) {
+                const double eps = A.eps[seg];
+                exact_step<F>(SP, J, W, eps, unbal ? 1.0 / (1.0 + eps / A.rho) : 1.0, ++seq);
+                ++it;
+                if (it == A.n_iter)
+                    break;
+                if (it == A.seg_end[seg])
+                    ++seg;
+                if (A.exact_only)
+                    continue;
+            } else if (start == kMoved) {
+                recentre<F>(SP, J, W);
+            }
+            const bool trial = start == kTrial;
+            const double mul_hi = trial ? kSumHi : kMulHi;
+            const double eps = A.eps[seg];
+            const double damp = unbal ? 1.0 / (1.0 + eps / A.rho) : 1.0;
+
+            // ---- P around the references ---------------------------------------
+            if (!trial && wc == 0 && rho < RW)
+                S.rl[lrow] = has ? W.rl : INFINITY;
+            if (t < 2) {
+                S.flag_row[t] = 0;
+                S.flag_all[t] = 0;
+            }
+            __syncthreads();
+            T v[TR][TC];
+            {
+                // the cost goes straight to P's registers, every load in
+                // flight, and is turned into P in place.  Columns past M and
+                // rows past nrow read a neighbour and vanish in the exponent
+                // (their references are +inf).  The scheduling barriers keep
+                // one row's addresses and temporaries live at a time, and the
+                // empty asm keeps the compiler from computing every row's
+                // address once, outside the loop over steps.
+                const char *C = static_cast<const char *>(J.C);
+                const char *keep = reinterpret_cast<const char *>(J.keep);
+                int last = nrow - 1, m = M;
+                asm volatile("" : "+s"(C), "+s"(keep), "+s"(last), "+s"(m));
+                const int h = LC == 64 ? 0 : lane >> 4;
+                constexpr int rs = LC == 64 ? 1 : 4;  // wave rows per r
+                uint32_t qo[TC];
+#pragma unroll
+                for (int k = 0; k < TC; ++k)
+                    qo[k] = (uint32_t)min(F::col(k, wc, lane), m - 1);
+#pragma unroll
+                for (int r = 0; r < TR; ++r) {
+                    const uint32_t ro = (uint32_t)min(wr * RW + rs * r + h, last) * (uint32_t)m;
+#pragma unroll
+                    for (int k = 0; k < TC; ++k)
+                        v[r][k] = *reinterpret_cast<const T *>(C + (ro + qo[k]) *
+                                                                       (uint32_t)sizeof(T));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (keep != nullptr) {
+                    constexpr int KR = TR < 4 ? TR : 4;  // rows in flight
+#pragma unroll
+                    for (int r0 = 0; r0 < TR; r0 += KR) {
+                        uint8_t kp[KR][TC];
+#pragma unroll
+                        for (int r = 0; r < KR && r0 + r < TR; ++r) {
+                            const uint32_t ro =
+                                (uint32_t)min(wr * RW + rs * (r0 + r) + h, last) * (uint32_t)m;
+#pragma unroll
+                            for (int k = 0; k < TC; ++k)
+                                kp[r][k] = (uint8_t)keep[ro + qo[k]];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int r = 0; r < KR && r0 + r < TR; ++r)
+#pragma unroll
+                            for (int k = 0; k < TC; ++k)
+                                v[r0 + r][k] = kp[r][k] ? v[r0 + r][k] : (T)INFINITY;
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                const U u(eps);
+                if (trial) {
+                    // row references: K at the row's smallest cost
+                    float mine = INFINITY;
+#pragma unroll
+                    for (int r = 0; r < TR; ++r) {
+                        float x = (float)v[r][0];
+#pragma unroll
+                        for (int k = 1; k < TC; ++k)
+                            x = fminf(x, (float)v[r][k]);
+                        x = fminf(x, dpp_full_f<kDppQuadXor1>(x));
+                        x = fminf(x, dpp_full_f<kDppQuadXor2>(x));
+                        x = fminf(x, dpp_full_f<kDppRowHalfMirror>(x));
+                        x = fminf(x, dpp_full_f<kDppRowMirror>(x));
+                        if constexpr (LC == 64) {
+                            float o;
+                            float y = row_swap16_pair(x, o);
+                            x = fminf(y, o);
+                            y = row_swap32_pair(x, o);
+                            x = fminf(y, o);
+                            mine = rho == r ? x : mine;
+                        } else {
+                            mine = (lane & 15) == r ? x : mine;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (rho < RW)
+                        S.rm[wc * R + lrow] = mine;
+                    __syncthreads();
+                    if (has) {
+#pragma unroll
+                        for (int w = 0; w < WC; ++w)
+                            mine = fminf(mine, S.rm[w * R + lrow]);
+                        W.rl = __builtin_isfinite(mine) ? u.kval((T)mine) : 0.0;
+                    }
+                    if (wc == 0 && rho < RW)
+                        S.rl[lrow] = has ? W.rl : INFINITY;
+                    __syncthreads();
+                }
+                double ck[TC];
+#pragma unroll
+                for (int k = 0; k < TC; ++k)
+                    ck[k] = S.c[F::col(k, wc, lane)];
+#pragma unroll
+                for (int r = 0; r < TR; ++r) {
+                    const double l = S.rl[wr * RW + rs * r + h];
+#pragma unroll
+                    for (int k = 0; k < TC; ++k) {
+                        v[r][k] = U::build((u.kval(v[r][k]) - l) - ck[k]);
+                        if (k % 4 == 3)
+                            __builtin_amdgcn_sched_barrier(0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            Row L = W;  // W is in memory (it is passed to the calls above)
+            // the thread's owned columns t + kc * 512: multiplier, its carried
+            // rounding, the marginal (balanced linear, else in log units), the
+            // reference
+            double cb[KC], cnu[KC], cref[KC];
+            float ceb[KC];
+            bool cdead[KC];
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) {
+                const int jl = t + kc * F::NT;
+                cb[kc] = S.bd[jl];
+                ceb[kc] = S.eb[jl];
+                cnu[kc] = S.nu[jl];
+                cdead[kc] = S.dead[jl] != 0;
+                cref[kc] = jl < cn ? S.c[j0 + jl] : 0.0;
+            }
+
+            // ---- steps from P until epsilon changes or one is refused ----------
+            for (int fp = 0;; fp ^= 1) {
+                double rsum = 0.0;  // the lane's row
+                {
+                    T bk[TC];
+#pragma unroll
+                    for (int k = 0; k < TC; ++k)
+                        bk[k] = S.b[F::col(k, wc, lane)];
+#pragma unroll
+                    for (int q = 0; q < (NV + 3) / 4; ++q) {
+                        T z[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if (4 * q + i >= NV) {
+                                z[i] = (T)0;
+                                continue;
+                            }
+                            if constexpr (LC == 64) {
+                                T s[4];
+#pragma unroll
+                                for (int x = 0; x < 4; ++x)
+                                    s[x] = v[4 * (4 * q + i) + x][0] * bk[0];
+#pragma unroll
+                                for (int k = 1; k < TC; ++k)
+#pragma unroll
+                                    for (int x = 0; x < 4; ++x)
+                                        s[x] = fma(v[4 * (4 * q + i) + x][k], bk[k], s[x]);
+                                z[i] = pair_swap16(pair_swap32(s[0], s[2]),
+                                                   pair_swap32(s[1], s[3]));
+                            } else {
+                                T s = v[4 * q + i][0] * bk[0];
+#pragma unroll
+                                for (int k = 1; k < TC; ++k)
+                                    s = fma(v[4 * q + i][k], bk[k], s);
+                                z[i] = s;
+                            }
+                        }
+                        const double x = row16_sum4(z, odd, odd2);
+                        rsum = ((lane >> 2) & 3) == q ? x : rsum;
+                    }
+                }
+                if constexpr (WC > 1) {
+                    if (rho < RW)
+                        S.rs[wc * R + lrow] = rsum;
+                    __syncthreads();
+                    rsum = 0.0;
+                    if (rho < RW) {
+#pragma unroll
+                        for (int w = 0; w < WC; ++w)
+                            rsum += S.rs[w * R + lrow];
+                    }
+                }
+                // the lane's row update, in each of the row's WC waves
+                double a_new, lu_new = L.lu;
+                float ea_new = 0.f;
+                T ah;
+                {
+                    if (!unbal) {
+                        a_new = L.mu * U::recip(rsum);
+                    } else {
+                        lu_new = damp * (L.lmu - (U::log_fast(rsum) + L.rl));
+                        a_new = U::exp_fast(lu_new + L.rl);
+                    }
+                    const bool ok = L.dead ? rsum == 0.0
+                                           : rsum >= kSumLo && rsum <= kSumHi && a_new <= mul_hi;
+                    if (L.dead || !has) {
+                        a_new = L.a;
+                        lu_new = L.lu;
+                    }
+                    if constexpr (PW == 1) {
+                        const double x = fma(a_new, (double)L.ea, a_new);
+                        ah = (float)x;
+                        if (ah != 0.f)
+                            ea_new = (float)(x - (double)ah) * __builtin_amdgcn_rcpf(ah);
+                    } else {
+                        ah = a_new;
+                    }
+                    if (ballot(has && !ok) != 0 && lane == 0)
+                        S.flag_row[fp] = 1;
+                }
+                {
+                    T cs[TC];
+#pragma unroll
+                    for (int k = 0; k < TC; ++k)
+                        cs[k] = (T)0;
+                    if constexpr (LC == 64) {
+#pragma unroll
+                        for (int r = 0; r < TR; ++r) {
+                            const T ar = readlane_t(ah, 16 * (r & 3) + (r >> 2));
+#pragma unroll
+                            for (int k = 0; k < TC; ++k)
+                                cs[k] = fma(v[r][k], ar, cs[k]);
+                        }
+#pragma unroll
+                        for (int k = 0; k < TC; ++k)
+                            S.cp[wr * CW + F::col(k, wc, lane)] = cs[k];
+                    } else {
+                        unroll<TR>([&](auto ri) {
+                            constexpr int r = decltype(ri)::value;
+                            const T ar = dpp_t<kDppRowNewBcast0 + r>(ah);
+#pragma unroll
+                            for (int k = 0; k < TC; ++k)
+                                cs[k] = fma(v[r][k], ar, cs[k]);
+                        });
+                        // the four groups' sums; each keeps a quarter of the
+                        // columns (a column without a partner is kept twice)
+                        constexpr int n1 = (TC + 1) / 2, n2 = (n1 + 1) / 2;
+                        T y[n1 + 1];
+#pragma unroll
+                        for (int p = 0; p < n1; ++p)
+                            y[p] = pair_swap32(cs[2 * p], cs[min(2 * p + 1, TC - 1)]);
+#pragma unroll
+                        for (int p = 0; p < n2; ++p) {
+                            const T z = pair_swap16(y[2 * p], y[min(2 * p + 1, n1 - 1)]);
+                            const int p1 = min(2 * p + ((lane >> 4) & 1), n1 - 1);
+                            const int k = min(2 * p1 + (lane >> 5), TC - 1);
+                            S.cp[wr * CW + F::col(k, wc, lane)] = z;
+                        }
+                    }
+                }
+                __syncthreads();
+                if (t == 0) {
+                    S.flag_row[fp ^ 1] = 0;
+                    S.flag_all[fp ^ 1] = 0;
+                }
+                uint32_t bad = (uint32_t)S.flag_row[fp];
+                int late = 0;
+                auto local_sum = [&](int j) {
+                    double s[WR];
+#pragma unroll
+                    for (int w = 0; w < WR; ++w)
+                        s[w] = (double)S.cp[w * CW + j];
+#pragma unroll
+                    for (int h = 1; h < WR; h *= 2)
+#pragma unroll
+                        for (int w = 0; w + h < WR; w += 2 * h)
+                            s[w] += s[w + h];
+                    return s[0];
+                };
+                uint32_t tag = 0;
+                // this exchange's slots; a word's byte offset in them fits 32
+                // bits (at most 256 workgroups x 2 words x 4096 columns x 8)
+                const char *pw = nullptr;
+                char *cw = nullptr;
+                const uint32_t prow = (uint32_t)(XW * Mp) * 8u;  // one workgroup's partials
+                // Sum of column j's partials of workgroups q0, q0 + step, ...
+                // (`per` of them, the last perhaps past G), in that order, N
+                // in flight at a time.  N is a constant and every load goes out
+                // unconditionally: behind branches they would be waited for
+                // one by one (about 1100 cycles each).
+                auto gather_n = [&](int j, int q0, int step, auto nc) {
+                    constexpr int N = decltype(nc)::value;
+                    const uint32_t o0 = (uint32_t)q0 * prow + (uint32_t)j * 8u;
+                    const uint32_t so = (uint32_t)step * prow;
+                    const int mine = q0 + (per - 1) * step < G ? per : per - 1;
+                    double acc = 0.0;
+                    for (int u0 = 0; u0 < per; u0 += N) {
+                        uint64_t w[N][PW];
+                        Waiter wt;
+                        for (;;) {
+                            uint32_t diff = 0;
+#pragma unroll
+                            for (int i = 0; i < N; ++i) {
+                                const uint32_t o =
+                                    u0 + i < mine ? o0 + (uint32_t)(u0 + i) * so : o0;
+#pragma unroll
+                                for (int p = 0; p < PW; ++p)
+                                    w[i][p] = get_word(reinterpret_cast<const uint64_t *>(
+                                        pw + (o + (uint32_t)(p * Mp) * 8u)));
+                            }
+#pragma unroll
+                            for (int i = 0; i < N; ++i)
+#pragma unroll
+                                for (int p = 0; p < PW; ++p)
+                                    diff |= (uint32_t)(w[i][p] >> 32) ^ tag;
+                            if (diff <= 1u) {
+                                bad |= diff;
+                                break;
+                            }
+                            if (!wt.more()) {
+                                late = 1;
+                                break;
+                            }
+                        }
+#pragma unroll
+                        for (int i = 0; i < N; ++i) {
+                            if constexpr (PW == 1)
+                                acc += (double)(u0 + i < mine
+                                                    ? __uint_as_float((uint32_t)w[i][0])
+                                                    : 0.f);
+                            else
+                                acc += u0 + i < mine
+                                           ? pack_d((uint32_t)w[i][0], (uint32_t)w[i][PW - 1])
+                                           : 0.0;
+                        }
+                    }
+                    return acc;
+                };
+                auto gather = [&](int j, int q0, int step) {
+                    if (per <= 2)
+                        return gather_n(j, q0, step, std::integral_constant<int, 2>{});
+                    if (per <= 4)
+                        return gather_n(j, q0, step, std::integral_constant<int, 4>{});
+                    return gather_n(j, q0, step, std::integral_constant<int, 8>{});
+                };
+                if constexpr (!SOLO) {
+                    ++seq;
+                    tag = seq << 1;
+                    pw = reinterpret_cast<const char *>(part + (size_t)(seq & 1) * G * XW * Mp);
+                    cw = reinterpret_cast<char *>(cast + (size_t)(seq & 1) * BW * Mp);
+                    char *mine = const_cast<char *>(pw) + (uint32_t)g * prow;
+#pragma unroll
+                    for (int kc = 0; kc < F::NK; ++kc) {
+                        const int j = t + kc * F::NT;
+                        if (j < M) {
+                            const double s = local_sum(j);
+                            uint64_t *p = reinterpret_cast<uint64_t *>(mine + (uint32_t)j * 8u);
+                            if constexpr (PW == 1) {
+                                put_word(p, __float_as_uint((float)s), tag | bad);
+                            } else {
+                                const uint64_t x = (uint64_t)__double_as_longlong(s);
+                                put_word(p, (uint32_t)x, tag | bad);
+                                put_word(p + Mp, (uint32_t)(x >> 32), tag | bad);
+                            }
+                        }
+                    }
+                    if (split > 1) {
+                        const int sp = t / cnp, jl = t % cnp;
+                        double acc = jl < cn ? gather(j0 + jl, sp, split) : 0.0;
+                        // groups within a wave add up over the lanes, the rest
+                        // in LDS
+                        if (cnp == 16)
+                            acc = pair_swap16(acc, acc);
+                        if (cnp <= 32)
+                            acc = pair_swap32(acc, acc);
+                        const int sub = cnp >= 64 ? sp : t >> 6;
+                        if (cnp >= 64 || lane < cnp)
+                            S.xs[sub * cnp + jl] = acc;
+                        if (bad & 1u)
+                            S.flag_row[fp] = 1;
+                        __syncthreads();
+                        bad |= (uint32_t)S.flag_row[fp];
+                    }
+                }
+                double b_new[KC];
+                float eb_new[KC];
+#pragma unroll
+                for (int kc = 0; kc < KC; ++kc) {
+                    const int jl = t + kc * F::NT;
+                    if (jl >= cn)
+                        break;
+                    const int j = j0 + jl;
+                    double s;
+                    if (SOLO) {
+                        s = local_sum(j);
+                    } else if (split > 1) {
+                        s = 0.0;
+                        for (int sub = 0; sub < min(split, F::NW); ++sub)
+                            s += S.xs[sub * cnp + jl];
+                    } else {
+                        s = gather(j, 0, 1);
+                    }
+                    double b;
+                    if (!unbal) {
+                        b = cnu[kc] * U::recip(s);
+                    } else {
+                        const double c = cref[kc];
+                        b = U::exp_fast(damp * (cnu[kc] - (U::log_fast(s) + c)) + c);
+                    }
+                    const bool ok = cdead[kc] ? s == 0.0
+                                              : s >= kSumLo && s <= kSumHi && b <= mul_hi;
+                    if (cdead[kc])
+                        b = cb[kc];
+                    bad |= ok ? 0u : 1u;
+                    b_new[kc] = b;
+                    eb_new[kc] = 0.f;
+                    T h;
+                    if constexpr (PW == 1) {
+                        const double x = fma(b, (double)ceb[kc], b);
+                        h = (float)x;
+                        if (h != 0.f)
+                            eb_new[kc] = (float)(x - (double)h) * __builtin_amdgcn_rcpf(h);
+                    } else {
+                        h = b;
+                    }
+                    S.b[j] = h;
+                    if (SOLO || direct)
+                        continue;
+                    if constexpr (!SOLO) {
+                        uint64_t *p = reinterpret_cast<uint64_t *>(cw + (uint32_t)j * 8u);
+                        if constexpr (PW == 1) {
+                            put_word(p, __float_as_uint(h), tag | (bad & 1u));
+                        } else {
+                            const uint64_t x = (uint64_t)__double_as_longlong(h);
+                            put_word(p, (uint32_t)x, tag | (bad & 1u));
+                            put_word(p + Mp, (uint32_t)(x >> 32), tag | (bad & 1u));
+                        }
+                    }
+                }
+                // every column's multiplier from its owner
+                auto gather_b = [&]() {
+                    constexpr int NK = F::NK;
+                    uint64_t w[NK][PW];
+                    Waiter wt;
+                    for (;;) {
+                        uint32_t diff = 0;
+#pragma unroll
+                        for (int kc = 0; kc < NK; ++kc)
+#pragma unroll
+                            for (int p = 0; p < PW; ++p)
+                                w[kc][p] = get_word(reinterpret_cast<const uint64_t *>(
+                                    cw + (uint32_t)(min(t + kc * F::NT, M - 1) + p * Mp) * 8u));
+#pragma unroll
+                        for (int kc = 0; kc < NK; ++kc)
+#pragma unroll
+                            for (int p = 0; p < PW; ++p)
+                                diff |= (uint32_t)(w[kc][p] >> 32) ^ tag;
+                        if (diff <= 1u)
+                            break;
+                        if (!wt.more()) {
+                            late = 1;
+                            break;
+                        }
+                    }
+#pragma unroll
+                    for (int kc = 0; kc < NK; ++kc) {
+                        bad |= (uint32_t)(w[kc][0] >> 32);
+                        const int j = t + kc * F::NT;
+                        if (j < M) {
+                            if constexpr (PW == 1)
+                                S.b[t + kc * F::NT] = __uint_as_float((uint32_t)w[kc][0]);
+                            else
+                                S.b[t + kc * F::NT] =
+                                    pack_d((uint32_t)w[kc][0], (uint32_t)w[kc][PW - 1]);
+                        }
+                    }
+                };
+                if constexpr (!SOLO) {
+                    if (!direct)
+                        gather_b();
+                }
+                if (bad & 1u)
+                    S.flag_all[fp] = 1;
+                if (late)
+                    S.abort = 1;
+                __syncthreads();
+                if (S.flag_all[fp] | S.abort) {
+                    // refused: the multipliers of the last accepted step again
+                    if (!direct) {
+                        ++seq;
+                        tag = seq << 1;
+                        cw = reinterpret_cast<char *>(cast + (size_t)(seq & 1) * BW * Mp);
+                    }
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc) {
+                        const int jl = t + kc * F::NT;
+                        if (jl >= cn)
+                            break;
+                        S.b[j0 + jl] = (T)cb[kc];
+                        if (!direct) {
+                            uint64_t *p = reinterpret_cast<uint64_t *>(cw + (uint32_t)(j0 + jl) * 8u);
+                            if constexpr (PW == 1) {
+                                put_word(p, __float_as_uint((float)cb[kc]), tag);
+                            } else {
+                                const uint64_t x = (uint64_t)__double_as_longlong(cb[kc]);
+                                put_word(p, (uint32_t)x, tag);
+                                put_word(p + Mp, (uint32_t)(x >> 32), tag);
+                            }
+                        }
+                    }
+                    if (!direct) {
+                        late = 0;
+                        gather_b();
+                        if (late)
+                            S.abort = 1;
+                    }
+                    start = kExact;
+                    break;
+                }
+#pragma unroll
+                for (int kc = 0; kc < KC; ++kc) {
+                    if (t + kc * F::NT < cn) {
+                        cb[kc] = b_new[kc];
+                        ceb[kc] = eb_new[kc];
+                    }
+                }
+                L.a = a_new;
+                L.ea = ea_new;
+                L.lu = lu_new;
+                L.derived = true;
+                ++it;
+                if (it == A.seg_end[seg] || trial) {
+                    if (it == A.seg_end[seg])
+                        ++seg;
+                    start = kMoved;
+                    break;
+                }
+            }
+            W = L;
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) {
+                S.bd[t + kc * F::NT] = cb[kc];
+                S.eb[t + kc * F::NT] = ceb[kc];
+            }
+            __syncthreads();
+        }
+        finish_problem<F>(SP, J, W, static_cast<T *>(A.log_u) + prob * A.N + i0,
+                          A.lu64 ? A.lu64 + prob * A.N + i0 : nullptr,
+                          static_cast<T *>(A.log_v) + prob * M,
+                          A.lv64 ? A.lv64 + prob * M : nullptr);
+    }
+}
+
+// ---- kernel addresses of a tile configuration -----------------------------------
+
+#define TM_KERNEL(T_, NW_, LC_, WC_, TC_, TR_, SOLO_) \
+    reinterpret_cast<const void *>(&sk_resident<Cfg<T_, NW_, LC_, WC_, TC_, TR_, SOLO_>>)
+#define TM_TILE(T_, NW_, LC_, WC_, TC_, TR_)                  \
+    {                                                         \
+        NW_, LC_, WC_, TC_, TR_,                              \
+            TM_KERNEL(T_, NW_, LC_, (WC_ > 2 ? 1 : WC_), TC_, TR_, true),     \
+            TM_KERNEL(T_, NW_, LC_, WC_, TC_, TR_, false)     \
+    }
+
+} // namespace
+} // namespace tmamd

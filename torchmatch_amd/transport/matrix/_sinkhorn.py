@@ -266,12 +266,14 @@ def _sinkhorn_divergence(  # noqa: PLR0913
 
     def ot(c, p, q, **checks):
         f, g = _potentials(c, p, q, eps, n_iter, scaling, **checks)
-        return (p * f).sum(dim=-1) + (q * g).sum(dim=-1)
+        # float64 sums: the divergence is a small difference of these values
+        return (p * f).sum(dim=-1, dtype=torch.float64) + (q * g).sum(
+            dim=-1, dtype=torch.float64)
 
     ot_ab = ot(cost, a, b, mask=mask, check_cost=check_cost, check_marginals=check_marginals)
     ot_aa = ot(_expand_self_cost(cost_aa, cost, batch, n), a, a)
     ot_bb = ot(_expand_self_cost(cost_bb, cost, batch, m), b, b)
-    return -(ot_ab - 0.5 * ot_aa - 0.5 * ot_bb)
+    return (0.5 * ot_aa + 0.5 * ot_bb - ot_ab).to(cost.dtype)
 
 
 def sinkhorn_divergence(  # noqa: PLR0913
