@@ -97,9 +97,14 @@ __device__ __forceinline__ void load_row_raw(const CostView &C, int i, float (&r
         raw[e] = src[min(e * 64 + lane, C.M - 1)];
 }
 
-// The padded-tile view of a raw cost: +inf -> sentinel, columns >= M -> 0.
+// The padded-tile view of a raw cost: +inf -> sentinel, columns >= M -> 0.  In
+// bit operations: as selects it compiles to two branches per value (a row of
+// eight chunks then took 1500 cycles in scan_group).
 __device__ __forceinline__ float fix_cost(const CostView &C, float raw, int j) {
-    return j >= C.M ? 0.f : (isfinite(raw) ? raw : C.sentinel);
+    const uint32_t u = __float_as_uint(raw), s = __float_as_uint(C.sentinel);
+    const uint32_t inf = (uint32_t)((int)(0x7f7fffffu - (u & 0x7fffffffu)) >> 31);
+    const uint32_t in = (uint32_t)((j - C.M) >> 31);
+    return __uint_as_float(((u & ~inf) | (s & inf)) & in);
 }
 
 // Row i of the padded tile into registers (values for j >= K are unused).
@@ -459,6 +464,202 @@ __device__ void scan_row(LDS &L, const CostView &C, int fi, int E, int K,
         L.cg[fi][lane] = lane == 0 ? g0 : (lane == 1 ? g1 : g2);
     }
     L.ctau[fi] = k4 == kKeyNone ? finf() : key_to_float(k4);  // every lane, the same word
+}
+
+// scan_dense over the rows that own the columns of a tied group, positions
+// [lo, hi) of cols[] and the columns that join it.  Returns the first position
+// not scanned: hi (advanced by the joins) when all were, less when a row brings
+// more than kGroupJoins joins, which the position-by-position scan takes in
+// bulk.  final_j: the unassigned column that ended the path, if one did.
+//
+// Only joins look at positions: a column's new d is the smallest of the rows'
+// values and its pred the first row of the group that reached it (strict '<'
+// in group order).  So lanes keep their columns e * 64 + lane with d, v and pred
+// in registers and rows are read coalesced, four in flight.  A value equal to
+// the group's level, below the column's d, ends the path at the first
+// unassigned such column in position order, or else joins: the joins of a row
+// are swapped to the group's end in position order, with ev[] holding every
+// column's position meanwhile.
+//
+// With N > M the N - M padding columns are one tied group that every path
+// scans, about 270 rows a path at (8, 500, 300) uniform: 40.2 ms position by
+// position, 16.3 ms with this (points 53.4 and 22.9).  A row is some 500 cycles
+// of this wave's own arithmetic (eight columns a lane) and a join on every
+// fourth row; one wave a problem is what bounds it.  Groups of kGroupScan or
+// more come here: the set-up reads the K columns once, as one row does (groups
+// of two at square sizes: no change either way).  Above kGroupJoins joins a
+// row, the ballots a chunk of the bulk path are fewer than the reductions here
+// ((8, 300, 500) of few whole values: 1.56 ms before, 1.40 now).
+constexpr int kGroupScan = 2;
+constexpr int kGroupJoins = 6;
+template <int NC, class LDS>
+__device__ __forceinline__ int scan_group(LDS &L, const CostView &C, int K, int lo, int &hi,
+                                          int &final_j) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int e = 0; e < NC; ++e)
+        if (e * 64 + lane < K)
+            L.ev[L.cols[e * 64 + lane]] = e * 64 + lane;
+    lds_sync();
+    // settled columns (and lanes past K) have v = -inf: their values are +inf
+    float d[NC], v[NC];
+    int pred[NC];
+    uint32_t off[NC], real[NC];  // byte in a row; all ones below M
+#pragma unroll
+    for (int e = 0; e < NC; ++e) {
+        const int j = min(e * 64 + lane, K - 1);
+        const bool open = e * 64 + lane < K && L.ev[j] >= hi;
+        d[e] = L.d[j];
+        v[e] = open ? L.v[j] : -INFINITY;
+        pred[e] = L.pred[j];
+        off[e] = 4u * (uint32_t)min(e * 64 + lane, C.M - 1);
+        real[e] = (uint32_t)((e * 64 + lane - C.M) >> 31);
+    }
+    auto load = [&](int i, float(&raw)[NC]) {
+        const char *src = reinterpret_cast<const char *>(C.src + (int64_t)min(i, C.N - 1) * C.M);
+#pragma unroll
+        for (int e = 0; e < NC; ++e)
+            raw[e] = *reinterpret_cast<const float *>(src + off[e]);
+    };
+    // One row of the group (owner i, shift hr, level lr): kNext, or kEnded, or
+    // kBulk (nothing of the row kept then; padding rows go there too).
+    enum { kNext, kEnded, kBulk };
+    auto scan_one = [&](const float(&raw)[NC], int i, float hr, float lr)
+                        __attribute__((always_inline)) -> int {
+        if (i >= C.N)
+            return kBulk;
+        float dn[NC], low = INFINITY;
+        int pn[NC];
+#pragma unroll
+        for (int e = 0; e < NC; ++e) {
+            const uint32_t u = __float_as_uint(raw[e]);
+            const uint32_t f = (u & 0x7f800000u) == 0x7f800000u ? __float_as_uint(C.sentinel) : u;
+            const float x = __uint_as_float(f & real[e]) - v[e] - hr;
+            pn[e] = x < d[e] ? i : pred[e];
+            dn[e] = fminf(x, d[e]);
+            low = fminf(low, x);
+        }
+        if (ballot(low <= lr) != 0) {
+            // a join has x == level below the old d: then pred is i and d the
+            // level (a row is scanned once a path, so no other column has both)
+            int open_at = kKeyNone, n_join = 0, one = 0;
+            uint32_t mine = 0;  // the lane's joining chunks
+#pragma unroll
+            for (int e = 0; e < NC; ++e) {
+                const bool in = dn[e] == lr && pn[e] == i;
+                const uint64_t m = ballot(in);
+                n_join += __popcll(m);
+                one = m != 0 ? e * 64 + first_lane(m) : one;
+                mine |= in ? 1u << e : 0u;
+            }
+            if (n_join > kGroupJoins)
+                return kBulk;
+            if (n_join == 1) {
+                const int p = L.ev[one], yj = L.y[one], other = L.cols[hi];
+                L.pred[one] = i;  // every lane writes the same words
+                if (uniform_i(yj) < 0) {
+                    final_j = one;
+                    return kEnded;
+                }
+                L.cols[p] = other;
+                L.ev[other] = p;
+                L.cols[hi] = one;
+                L.ev[one] = hi;
+                L.d[one] = lr;
+                ++hi;
+#pragma unroll
+                for (int e = 0; e < NC; ++e)
+                    v[e] = one == e * 64 + lane ? -INFINITY : v[e];
+                lds_sync();
+            } else if (n_join > 1) {
+                for (uint32_t m = mine; m != 0; m &= m - 1) {
+                    const int j = __builtin_ctz(m) * 64 + lane;
+                    if (L.y[j] < 0)
+                        open_at = min(open_at, L.ev[j]);
+                }
+                open_at = wave_min_key_s(open_at);
+                if (open_at != kKeyNone) {
+                    final_j = L.cols[open_at];
+                    L.pred[final_j] = i;
+                    return kEnded;
+                }
+                for (int k = 0; k < n_join; ++k) {
+                    int p = kKeyNone;
+                    for (uint32_t m = mine; m != 0; m &= m - 1)
+                        p = min(p, L.ev[__builtin_ctz(m) * 64 + lane]);
+                    p = wave_min_key_s(p);
+                    const int j = uniform_i(L.cols[p]);
+                    const int other = uniform_i(L.cols[hi]);
+                    L.cols[p] = other;
+                    L.ev[other] = p;
+                    L.cols[hi] = j;
+                    L.ev[j] = hi;
+                    L.d[j] = lr;
+                    L.pred[j] = i;
+                    ++hi;
+                    if ((j & 63) == lane)
+                        mine &= ~(1u << (j >> 6));
+#pragma unroll
+                    for (int e = 0; e < NC; ++e)
+                        v[e] = j == e * 64 + lane ? -INFINITY : v[e];
+                    lds_sync();
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < NC; ++e) {
+            d[e] = dn[e];
+            pred[e] = pn[e];
+        }
+        return kNext;
+    };
+    constexpr int D = NC <= 16 ? 4 : 2;  // rows in flight
+    int done = lo, st = kNext;
+    while (done < hi) {
+        // the next 64 members: owner row, level and shift h of each
+        const int jq = L.cols[min(done + lane, hi - 1)];
+        const int iq = L.y[jq];
+        const float level = L.d[jq];
+        float cq = C.src[(int64_t)min(iq, C.N - 1) * C.M + min(jq, C.M - 1)];
+        cq = iq < C.N ? fix_cost(C, cq, jq) : 0.f;
+        const float h = cq - L.v[jq] - level;
+        const int n = min(64, hi - done);
+        float raw[D][NC];
+#pragma unroll
+        for (int b = 0; b < D; ++b)
+            load(readlane_i(iq, min(b, n - 1)), raw[b]);
+        for (int r0 = 0; r0 < n; r0 += D) {
+#pragma unroll
+            for (int b = 0; b < D; ++b) {
+                const int r = r0 + b;
+                if (r >= n)
+                    break;
+                st = scan_one(raw[b], readlane_i(iq, r), readlane_f(h, r), readlane_f(level, r));
+                if (st != kNext) {
+                    done += r;
+                    goto out;
+                }
+                // (past the window the last row again: every turn issues the same loads)
+                load(readlane_i(iq, min(r + D, n - 1)), raw[b]);
+            }
+        }
+        done += n;
+    }
+out:
+    if (st == kEnded) {
+        lds_sync();
+        return done;
+    }
+#pragma unroll
+    for (int e = 0; e < NC; ++e) {
+        const int j = e * 64 + lane;
+        if (j < K && v[e] > -INFINITY) {
+            L.d[j] = d[e];
+            L.pred[j] = pred[e];
+        }
+    }
+    lds_sync();
+    return done;
 }
 
 // ---- prefill: the column reduction's minima and every row's cache -----------
@@ -1405,7 +1606,11 @@ __device__ __forceinline__ bool large_solve(const int K, const int E, LDS &L, co
             // scan_dense
             int slo = lo, shi = hi;
             bool early = false;
-            while (slo != shi) {
+            if (shi - slo >= kGroupScan) {
+                slo = scan_group<NC>(L, C, K, slo, shi, final_j);
+                early = final_j >= 0;
+            }
+            while (slo != shi && !early) {
                 const int q = slo++;
                 const int jq = L.cols[q];
                 const int iq = L.y[jq];
