@@ -121,6 +121,21 @@ def test_float64(B, N, M, rho, device):
     assert sk_parity.logp_err(got, ref) <= 2e-13
 
 
+@pytest.mark.parametrize(("B", "N", "M"), [
+    (1, 1810, 43), (51, 634, 42), (1, 2000, 17), (2, 700, 5), (1, 1500, 1), (1, 700, 100)])
+def test_fewer_workgroups_than_merge_groups(B, N, M, device):
+    """Narrow and tall: the threads that merge a column are more than the
+    workgroups that have a partial of it (all but the last shape)."""
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=N + M)
+    _check(f"{(B, N, M)}", cost, workloads.dirichlet(B, N, seed=1),
+           workloads.dirichlet(B, M, seed=2), 0.05, 20, device)
+
+
+@pytest.mark.parametrize(("B", "N", "M"), [(2, 900, 7), (1, 1200, 40), (1, 600, 60)])
+def test_fewer_workgroups_than_merge_groups_float64(B, N, M, device):
+    test_float64(B, N, M, None, device)
+
+
 @pytest.mark.parametrize(("B", "N", "M"), [(5, 120, 1028), (2, 300, 200)])
 def test_streaming_groups_same_bits(B, N, M, device, monkeypatch):
     """The streaming step (which serves captures and matrices too large for the

@@ -1054,7 +1054,8 @@ sk_resident(const ResArgs A) {
                     }
                     if (split > 1) {
                         const int sp = t / cnp, jl = t % cnp;
-                        double acc = jl < cn ? gather(j0 + jl, sp, split) : 0.0;
+                        // (fewer workgroups than groups: the rest have no partial)
+                        double acc = jl < cn && sp < G ? gather(j0 + jl, sp, split) : 0.0;
                         // groups within a wave add up over the lanes, the rest
                         // in LDS
                         if (cnp == 16)
