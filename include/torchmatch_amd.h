@@ -260,9 +260,9 @@ int tm_sinkhorn_read_stats(const void *workspace, int64_t B, int64_t N, int64_t 
  *   log_plan   device (B, N, M) output, may be NULL to skip the plan
  *   log_u, log_v  device (B, N), (B, M) outputs: the final scaling
  *              potentials (f = -eps * log_u, g = -eps * log_v)
- * Matrices that fit the chip's registers are solved in one launch (cooperative
- * when several workgroups share a problem; a `stream` under graph capture takes
- * the streaming steps).  Otherwise, with B >= 2, the steps of part of the batch
+ * Matrices that fit the chip's registers are solved in one launch where the form
+ * (below) allows it (cooperative when several workgroups share a problem; a
+ * `stream` under graph capture takes the streaming steps).  Otherwise, with B >= 2, the steps of part of the batch
  * run on a side stream of the library's own (created on the first such call per
  * device of `stream`, default priority), forked and joined with events:
  * the call stays stream-ordered on `stream`.  TORCHMATCH_AMD_SINKHORN_GROUPS=1
@@ -275,6 +275,26 @@ int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, int64_t B, i
                             int64_t M, const double *eps_sched, int32_t n_iter, double rho,
                             float k_eps, float *log_plan, float *log_u, float *log_v,
                             void *workspace, size_t workspace_bytes, hipStream_t stream);
+
+/* What the caller reads of a solve.  With TM_SK_PLAN, log_u and log_v may
+ * differ from the plain calls' by a constant moved from one to the other
+ * (float32: up to 3e-4 of their norm, float64: 5e-14), which the plan does
+ * not show; every shape that fits the chip's
+ * registers is then solved in one launch.  TM_SK_POTENTIALS (the plain calls)
+ * does so only for float32 shapes whose steps carry float64 potentials (rows
+ * of 128 columns and more, a multiple of four), TM_SK_STEPS never. */
+enum { TM_SK_POTENTIALS = 0, TM_SK_PLAN = 1, TM_SK_STEPS = 2 };
+
+/* The two halves with a form; give both the same. */
+int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *keep, const float *a,
+                                 const float *b, int64_t B, int64_t N, int64_t M, float k_eps,
+                                 int32_t form, void *workspace, size_t workspace_bytes,
+                                 hipStream_t stream);
+int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *keep, int64_t B, int64_t N,
+                                 int64_t M, const double *eps_sched, int32_t n_iter, double rho,
+                                 float k_eps, int32_t form, float *log_plan, float *log_u,
+                                 float *log_v, void *workspace, size_t workspace_bytes,
+                                 hipStream_t stream);
 
 /* Both halves without a mask and without reading the statistics back: the
  * cost must hold no NaN / -inf and the marginals must be non-negative.
@@ -301,6 +321,12 @@ int tm_sinkhorn_f64(const double *cost, const double *a, const double *b, int64_
                     int64_t N, int64_t M, const double *eps_sched, int32_t n_iter, double rho,
                     double *log_plan, double *log_u, double *log_v, void *workspace,
                     size_t workspace_bytes, hipStream_t stream);
+/* The same with a form (TM_SK_PLAN: one launch where the matrix fits). */
+int tm_sinkhorn_form_f64(const double *cost, const double *a, const double *b, int64_t B,
+                         int64_t N, int64_t M, const double *eps_sched, int32_t n_iter,
+                         double rho, int32_t form, double *log_plan, double *log_u,
+                         double *log_v, void *workspace, size_t workspace_bytes,
+                         hipStream_t stream);
 
 #ifdef __cplusplus
 }

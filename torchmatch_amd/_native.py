@@ -93,6 +93,29 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
             _VP, _VP, _VP, _VP, ctypes.c_size_t, _VP,
         ],
     ),
+    "tm_sinkhorn_prepare_form_f32": (
+        ctypes.c_int,
+        [
+            _VP, _VP, _VP, _VP, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+            ctypes.c_float, ctypes.c_int32, _VP, ctypes.c_size_t, _VP,
+        ],
+    ),
+    "tm_sinkhorn_iterate_form_f32": (
+        ctypes.c_int,
+        [
+            _VP, _VP, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+            ctypes.POINTER(ctypes.c_double), ctypes.c_int32, ctypes.c_double, ctypes.c_float,
+            ctypes.c_int32, _VP, _VP, _VP, _VP, ctypes.c_size_t, _VP,
+        ],
+    ),
+    "tm_sinkhorn_form_f64": (
+        ctypes.c_int,
+        [
+            _VP, _VP, _VP, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+            ctypes.POINTER(ctypes.c_double), ctypes.c_int32, ctypes.c_double, ctypes.c_int32,
+            _VP, _VP, _VP, _VP, ctypes.c_size_t, _VP,
+        ],
+    ),
     "tm_sinkhorn_f32": (
         ctypes.c_int,
         [

@@ -1890,9 +1890,23 @@ int launch_plan64(const SinkhornLayout &L, const FusedPtrs &P, const float *cost
     return TM_OK;
 }
 
+// Whether a call of this form runs resident (where the launch can).  Balanced
+// potentials hold a neutral mode (a constant moved from log_u to log_v) that
+// every step's rounding feeds: the two-sweep step's natural-unit float32
+// potentials end up to 3e-4 of their norm from the float64 iteration's, the
+// fused step's and the resident solve's within 5e-7.  A caller that reads the
+// potentials gets those of the step its shape has always had, so the resident
+// solve takes such a call on the fused step's shapes only; plans, where
+// the constant cancels, differ by 1e-7 and take it everywhere.
+bool resident_form(const SinkhornLayout &L, int32_t form) {
+    return L.res.cfg >= 0 &&
+           (form == TM_SK_PLAN || (form == TM_SK_POTENTIALS && L.fused != kFzNone));
+}
+
 // Not under capture: a cooperative launch cannot be recorded.
-bool resident_ok(const SinkhornLayout &L, const void *workspace, hipStream_t stream) {
-    return L.res.cfg >= 0 && ((uintptr_t)workspace % 16) == 0 && !stream_capturing(stream);
+bool resident_ok(const SinkhornLayout &L, int32_t form, const void *workspace,
+                 hipStream_t stream) {
+    return resident_form(L, form) && ((uintptr_t)workspace % 16) == 0 && !stream_capturing(stream);
 }
 
 } // namespace
@@ -1901,6 +1915,15 @@ extern "C" int tm_sinkhorn_prepare_f32(const float *cost, const uint8_t *keep, c
                                        const float *b, int64_t B, int64_t N, int64_t M,
                                        float k_eps, void *workspace, size_t workspace_bytes,
                                        hipStream_t stream) {
+    return tm_sinkhorn_prepare_form_f32(cost, keep, a, b, B, N, M, k_eps, TM_SK_POTENTIALS,
+                                        workspace, workspace_bytes, stream);
+}
+
+extern "C" int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *keep,
+                                            const float *a, const float *b, int64_t B, int64_t N,
+                                            int64_t M, float k_eps, int32_t form,
+                                            void *workspace, size_t workspace_bytes,
+                                            hipStream_t stream) {
     if (B < 0 || N < 0 || M < 0 || !(k_eps >= 0.f))
         return TM_ERR_INVALID_ARGUMENT;
     if (B == 0 || N == 0 || M == 0)
@@ -1926,7 +1949,7 @@ extern "C" int tm_sinkhorn_prepare_f32(const float *cost, const uint8_t *keep, c
     const int64_t n_flags = B * N > B * M ? B * N : B * M;
     TM_LAUNCH(sk_reset_flags, dim3(grid_for(n_flags, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
               stream, inf_row, B * N, inf_col, B * M, stats);
-    const bool resident = resident_ok(L, workspace, stream);
+    const bool resident = resident_ok(L, form, workspace, stream);
     const bool state64 = L.fused != kFzNone || L.res.cfg >= 0;
     double *mu64 = state64 ? reinterpret_cast<double *>(ws + L.off_mu64) : nullptr;
     double *nu64 = state64 ? reinterpret_cast<double *>(ws + L.off_nu64) : nullptr;
@@ -2001,6 +2024,17 @@ extern "C" int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, i
                                        int32_t n_iter, double rho, float k_eps, float *log_plan,
                                        float *log_u, float *log_v, void *workspace,
                                        size_t workspace_bytes, hipStream_t stream) {
+    return tm_sinkhorn_iterate_form_f32(cost, keep, B, N, M, eps_sched, n_iter, rho, k_eps,
+                                        TM_SK_POTENTIALS, log_plan, log_u, log_v, workspace,
+                                        workspace_bytes, stream);
+}
+
+extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *keep, int64_t B,
+                                            int64_t N, int64_t M, const double *eps_sched,
+                                            int32_t n_iter, double rho, float k_eps,
+                                            int32_t form, float *log_plan, float *log_u,
+                                            float *log_v, void *workspace,
+                                            size_t workspace_bytes, hipStream_t stream) {
     if (B < 0 || N < 0 || M < 0 || n_iter < 1 || eps_sched == nullptr || !(k_eps >= 0.f))
         return TM_ERR_INVALID_ARGUMENT;
     for (int32_t s = 0; s < n_iter; ++s)
@@ -2038,7 +2072,7 @@ extern "C" int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, i
     const bool vec = (M % 4) == 0 && ((uintptr_t)log_v % 16) == 0;
     const bool fused = fused_ok(L, workspace);
 
-    if (resident_ok(L, workspace, stream)) {
+    if (resident_ok(L, form, workspace, stream)) {
         const FusedPtrs P = fused_ptrs(L, ws, log_u, log_v, 0);
         const SkResidentIo io{cost, keep, P.mu64, P.nu64, log_u, log_v, P.lu64, P.lv64,
                               ws + L.off_xch};
@@ -2051,7 +2085,7 @@ extern "C" int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, i
         if (rc != TM_ERR_UNSUPPORTED_SHAPE)
             return rc;
     }
-    if (L.res.cfg >= 0)
+    if (resident_form(L, form))
         k_eps = 0.f;  // the preparation pass left K to this call
 
     TM_LAUNCH(sk_fill, dim3(grid_for(B * N, kMapBlock, 1 << 30)), dim3(kMapBlock), 0, stream,

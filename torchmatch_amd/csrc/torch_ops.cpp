@@ -180,7 +180,8 @@ const uint8_t *keep_ptr(const c10::optional<at::Tensor> &keep) {
 // synchronisation; an empty tensor otherwise.
 std::tuple<at::Tensor, at::Tensor>
 sinkhorn_prepare_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &keep,
-                     const at::Tensor &a, const at::Tensor &b, double k_eps, bool read_stats) {
+                     const at::Tensor &a, const at::Tensor &b, double k_eps, bool read_stats,
+                     int64_t form) {
     TORCH_CHECK(cost.is_cuda() && a.is_cuda() && b.is_cuda(),
                 "sinkhorn: cost, a and b must be CUDA tensors");
     TORCH_CHECK(cost.dim() == 3, "sinkhorn: cost must be 3D (B, N, M)");
@@ -199,9 +200,10 @@ sinkhorn_prepare_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &ke
     const hipStream_t stream = current_stream(cost);
     if (read_stats)
         check_not_capturing(stream, "the transport Sinkhorn input check");
-    int rc = tm_sinkhorn_prepare_f32(cost.data_ptr<float>(), keep_ptr(keep), a.data_ptr<float>(),
-                                     b.data_ptr<float>(), B, N, M, (float)k_eps, ws.data_ptr(),
-                                     ws_bytes, stream);
+    int rc = tm_sinkhorn_prepare_form_f32(cost.data_ptr<float>(), keep_ptr(keep),
+                                          a.data_ptr<float>(), b.data_ptr<float>(), B, N, M,
+                                          (float)k_eps, (int32_t)form, ws.data_ptr(), ws_bytes,
+                                          stream);
     check_rc(rc, "sinkhorn_prepare");
     at::Tensor stats = at::empty({0}, at::TensorOptions().dtype(at::kDouble));
     if (read_stats) {
@@ -223,7 +225,7 @@ sinkhorn_prepare_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &ke
 std::tuple<at::Tensor, at::Tensor, at::Tensor>
 sinkhorn_iterate_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &keep,
                      const at::Tensor &ws, at::ArrayRef<double> eps_sched, double rho,
-                     double k_eps, bool write_plan) {
+                     double k_eps, bool write_plan, int64_t form) {
     TORCH_CHECK(cost.is_cuda() && ws.is_cuda(), "sinkhorn: cost and workspace must be CUDA tensors");
     TORCH_CHECK(cost.dim() == 3 && cost.scalar_type() == at::kFloat && cost.is_contiguous(),
                 "sinkhorn: cost must be a contiguous float32 (B, N, M) tensor");
@@ -237,9 +239,9 @@ sinkhorn_iterate_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &ke
                                      : at::empty({0}, cost.options());
     if (B == 0)
         return {log_plan, log_u, log_v};
-    const int rc = tm_sinkhorn_iterate_f32(
+    const int rc = tm_sinkhorn_iterate_form_f32(
         cost.data_ptr<float>(), keep_ptr(keep), B, N, M, eps_sched.data(),
-        (int32_t)eps_sched.size(), rho, (float)k_eps,
+        (int32_t)eps_sched.size(), rho, (float)k_eps, (int32_t)form,
         write_plan ? log_plan.data_ptr<float>() : nullptr, log_u.data_ptr<float>(),
         log_v.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), current_stream(cost));
     check_rc(rc, "sinkhorn_iterate");
@@ -252,7 +254,7 @@ sinkhorn_iterate_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &ke
 // write_plan is false.
 std::tuple<at::Tensor, at::Tensor, at::Tensor>
 sinkhorn_f64_hip(const at::Tensor &cost, const at::Tensor &a, const at::Tensor &b,
-                 at::ArrayRef<double> eps_sched, double rho, bool write_plan) {
+                 at::ArrayRef<double> eps_sched, double rho, bool write_plan, int64_t form) {
     TORCH_CHECK(cost.is_cuda() && a.is_cuda() && b.is_cuda(),
                 "sinkhorn: cost, a and b must be CUDA tensors");
     TORCH_CHECK(cost.dim() == 3 && cost.scalar_type() == at::kDouble && cost.is_contiguous(),
@@ -271,13 +273,34 @@ sinkhorn_f64_hip(const at::Tensor &cost, const at::Tensor &a, const at::Tensor &
                                      : at::empty({0}, cost.options());
     const size_t ws_bytes = tm_sinkhorn_f64_workspace_bytes(B, N, M);
     auto ws = at::empty({(int64_t)(ws_bytes > 0 ? ws_bytes : 1)}, cost.options().dtype(at::kByte));
-    const int rc = tm_sinkhorn_f64(
+    const int rc = tm_sinkhorn_form_f64(
         cost.data_ptr<double>(), a.data_ptr<double>(), b.data_ptr<double>(), B, N, M,
-        eps_sched.data(), (int32_t)eps_sched.size(), rho,
+        eps_sched.data(), (int32_t)eps_sched.size(), rho, (int32_t)form,
         write_plan ? log_plan.data_ptr<double>() : nullptr, log_u.data_ptr<double>(),
         log_v.data_ptr<double>(), ws.data_ptr(), ws_bytes, current_stream(cost));
     check_rc(rc, "sinkhorn_f64");
     return {log_plan, log_u, log_v};
+}
+
+// The ops without a form: every output counts.
+std::tuple<at::Tensor, at::Tensor>
+sinkhorn_prepare_plain(const at::Tensor &cost, const c10::optional<at::Tensor> &keep,
+                       const at::Tensor &a, const at::Tensor &b, double k_eps, bool read_stats) {
+    return sinkhorn_prepare_hip(cost, keep, a, b, k_eps, read_stats, TM_SK_POTENTIALS);
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor>
+sinkhorn_iterate_plain(const at::Tensor &cost, const c10::optional<at::Tensor> &keep,
+                       const at::Tensor &ws, at::ArrayRef<double> eps_sched, double rho,
+                       double k_eps, bool write_plan) {
+    return sinkhorn_iterate_hip(cost, keep, ws, eps_sched, rho, k_eps, write_plan,
+                                TM_SK_POTENTIALS);
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor>
+sinkhorn_f64_plain(const at::Tensor &cost, const at::Tensor &a, const at::Tensor &b,
+                   at::ArrayRef<double> eps_sched, double rho, bool write_plan) {
+    return sinkhorn_f64_hip(cost, a, b, eps_sched, rho, write_plan, TM_SK_POTENTIALS);
 }
 
 } // namespace
@@ -296,10 +319,20 @@ TORCH_LIBRARY(torchmatch_amd, m) {
           "float rho, float k_eps, bool write_plan) -> (Tensor, Tensor, Tensor)");
     m.def("sinkhorn_f64(Tensor cost, Tensor a, Tensor b, float[] eps_sched, float rho, "
           "bool write_plan) -> (Tensor, Tensor, Tensor)");
+    // with the form of the call (TM_SK_* in torchmatch_amd.h)
+    m.def("sinkhorn_prepare.form(Tensor cost, Tensor? keep, Tensor a, Tensor b, float k_eps, "
+          "bool read_stats, int form) -> (Tensor, Tensor)");
+    m.def("sinkhorn_iterate.form(Tensor cost, Tensor? keep, Tensor ws, float[] eps_sched, "
+          "float rho, float k_eps, bool write_plan, int form) -> (Tensor, Tensor, Tensor)");
+    m.def("sinkhorn_f64.form(Tensor cost, Tensor a, Tensor b, float[] eps_sched, float rho, "
+          "bool write_plan, int form) -> (Tensor, Tensor, Tensor)");
 }
 
 TORCH_LIBRARY_IMPL(torchmatch_amd, CUDA, m) {
-    m.impl("sinkhorn_prepare", &sinkhorn_prepare_hip);
-    m.impl("sinkhorn_iterate", &sinkhorn_iterate_hip);
-    m.impl("sinkhorn_f64", &sinkhorn_f64_hip);
+    m.impl("sinkhorn_prepare", &sinkhorn_prepare_plain);
+    m.impl("sinkhorn_iterate", &sinkhorn_iterate_plain);
+    m.impl("sinkhorn_f64", &sinkhorn_f64_plain);
+    m.impl("sinkhorn_prepare.form", &sinkhorn_prepare_hip);
+    m.impl("sinkhorn_iterate.form", &sinkhorn_iterate_hip);
+    m.impl("sinkhorn_f64.form", &sinkhorn_f64_hip);
 }

@@ -13,6 +13,8 @@ from enum import Enum
 import torch
 
 from torchmatch_amd.transport.matrix._sinkhorn import (
+    FORM_PLAN,
+    FORM_STEPS,
     _device_checkable,
     _log_sinkhorn,
     _sinkhorn_divergence,
@@ -114,8 +116,12 @@ def solve(  # noqa: PLR0913, PLR0911
         return _out(res)
 
     # UNBALANCED_SINKHORN
+    # the duals below are differences of log masses of the plan, which show its
+    # last bits (up to 3e-5 of their value at reg 0.02): they stay those of the
+    # streaming steps
     log_plan = _unbalanced_sinkhorn(
-        cost, eps=reg, n_iter=n_iter, rho=rho, a=a_, b=b_, scaling=scaling, **checks
+        cost, eps=reg, n_iter=n_iter, rho=rho, a=a_, b=b_, scaling=scaling,
+        form=FORM_STEPS if unpack else FORM_PLAN, **checks
     )
     if not unpack:
         return _out(log_plan)
