@@ -123,6 +123,41 @@ def test_float64(B, N, M, rho, device):
     assert sk_parity.logp_err(got, ref) <= 2e-13
 
 
+@pytest.mark.parametrize("mode", [None, "exact"])
+@pytest.mark.parametrize("where", ["row", "column", "both"])
+@pytest.mark.parametrize(("B", "N", "M", "dtype", "far"), [
+    (2, 60, 90, "float64", 1e9), (2, 60, 90, "float64", 1e13), (1, 400, 300, "float64", 1e11),
+    (1, 200, 1000, "float64", 1e9), (2, 60, 90, "float32", 1e8), (1, 400, 1200, "float32", 1e8)])
+def test_far_row_and_column(B, N, M, dtype, far, where, mode, device, monkeypatch):
+    """A row and a column of finite costs so large (|C| / eps of 3e9 and more)
+    that a maximum held in float32 misses the sum by more than exp's range.
+    Epsilon is a power of two, the same in both types."""
+    if mode:
+        monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_RESIDENT", mode)
+    eps, dt = 2.0 ** -5, getattr(torch, dtype)
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=M).to(dt)
+    if where != "column":
+        cost[:, 3, :] = far
+    if where != "row":
+        cost[:, :, 7] = far
+    a, b = workloads.dirichlet(B, N, seed=1).to(dt), workloads.dirichlet(B, M, seed=2).to(dt)
+    ref = sk.log_sinkhorn_plan(cost.double(), eps=eps, n_iter=10, a=a.double(), b=b.double(),
+                               dtype=torch.float64)[0]
+    got = solve(cost.to(device), a=a.to(device), b=b.to(device), reg=eps, n_iter=10)
+    if dtype == "float32":  # entries of a far row or column that carry no mass
+        got = got.double().cpu()
+        none = ref < -1e6
+        assert ((got - ref).abs()[none] <= 2.0 ** -23 * ref.abs()[none]).all()
+        got[none] = ref[none]
+    err = sk_parity.logp_err(got, ref)
+    # a few float64 roundings of |C| / eps in each of the two, over the float32
+    # tests' bound or test_float64's
+    bound = 16 * 2.0 ** -52 * far / eps + (sk_parity.ELEM_BOUND if dtype == "float32" else 2e-13)
+    print(f"far {(B, N, M)} {dtype} {far:.0e} {where} {mode}: {err:.2e}, bound {bound:.2e}",
+          flush=True)
+    assert err <= bound
+
+
 @pytest.mark.parametrize(("B", "N", "M"), [
     (1, 1810, 43), (51, 634, 42), (1, 2000, 17), (2, 700, 5), (1, 1500, 1), (1, 700, 100)])
 def test_fewer_workgroups_than_merge_groups(B, N, M, device):

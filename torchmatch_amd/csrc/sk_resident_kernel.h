@@ -111,6 +111,15 @@ template <> struct Unit<double> {
 
 __device__ __forceinline__ double shift_of(double m) { return isinf(m) ? 0.0 : m; }
 
+// Doubles as integers of the same order (for an integer maximum in LDS).
+__device__ __forceinline__ uint64_t order_key(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    return (u >> 63) != 0 ? ~u : u | (1ull << 63);
+}
+__device__ __forceinline__ double of_order_key(uint64_t k) {
+    return __longlong_as_double((long long)((k >> 63) != 0 ? k & ~(1ull << 63) : ~k));
+}
+
 __device__ __forceinline__ double pack_d(uint32_t lo, uint32_t hi) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
@@ -234,7 +243,7 @@ template <typename T, int NW_, int LC_, int WC_, int TC_, int TR_, bool SOLO_> s
     static constexpr int NK = (CW + NT - 1) / NT;          // columns per thread
     static constexpr int KC = SOLO ? NK : 1;               // owned columns per thread
     static constexpr int PW = Unit<T>::kPartWords;  // words of a column partial
-    static constexpr int XW = PW + 1;               // words of an exact partial (max, sum)
+    static constexpr int XW = PW + 2;               // words of an exact partial (max, sum)
     static constexpr int BW = PW + 2;               // words of an exact broadcast (c, b)
     static_assert(RW <= 64 && RW % 4 == 0, "one row per lane");
     static __device__ __forceinline__ int col(int k, int wc, int lane) {
@@ -250,10 +259,10 @@ template <typename F> struct Shared {
     double xs[F::NT];              // split column sums
     double bd[F::KC * F::NT];        // owned columns: multiplier and marginal
     double nu[F::KC * F::NT];        // (unbalanced: in log units)
+    double rm[F::WC * F::R];       // exact step: row maxima
+    uint64_t cm[F::CW];            // exact step: column maxima (order_key)
     T b[F::CW];
     T cp[F::WR * F::CW];           // column sums of each row wave
-    float cm[F::WR * F::CW];       // exact step: their maxima
-    float rm[F::WC * F::R];        // exact step: row maxima
     float eb[F::KC * F::NT];
     uint8_t dead[F::KC * F::NT];
     int flag_row[2], flag_all[2], abort;
@@ -316,6 +325,8 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     const int wr = wid / WC, wc = wid % WC;
     const int M = J.M, Mp = J.Mp, G = J.G;
     const U u(eps);
+    for (int j = t; j < CW; j += F::NT)
+        S->cm[j] = order_key(-INFINITY);
     {
         double lvk[TC];
 #pragma unroll
@@ -332,13 +343,13 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
 #pragma unroll
             for (int r = 0; r < RG; ++r) {
                 double x[TC];
-                float m = -INFINITY;
+                double m = -INFINITY;
 #pragma unroll
                 for (int k = 0; k < TC; ++k) {
                     x[k] = u.kval(c[r][k]) + lvk[k];
-                    m = fmaxf(m, (float)x[k]);
+                    m = fmax(m, x[k]);
                 }
-                m = wave_max_all(m);
+                m = wave_max_all_d(m);
                 const double sh = shift_of(m);
                 double s = 0.0;
 #pragma unroll
@@ -357,10 +368,10 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     const int rho = lane_row(lane), row = wr * TR + rho;
     const bool has = rho < TR && row < J.nrow;
     if (has) {
-        float m = S->rm[row];
+        double m = S->rm[row];
 #pragma unroll
         for (int w = 1; w < WC; ++w)
-            m = fmaxf(m, S->rm[w * R + row]);
+            m = fmax(m, S->rm[w * R + row]);
         const double sh = shift_of(m);
         double s = 0.0;
 #pragma unroll
@@ -383,7 +394,7 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
         S->rl[row] = has ? W.lu : -INFINITY;
     __syncthreads();
     {
-        float m[TC];
+        double m[TC];
         T s[TC];
 #pragma unroll
         for (int k = 0; k < TC; ++k) {
@@ -401,9 +412,18 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
                 const double l = S->rl[wr * TR + r0 + r];
 #pragma unroll
                 for (int k = 0; k < TC; ++k)
-                    m[k] = fmaxf(m[k], (float)(u.kval(c[r][k]) + l));
+                    m[k] = fmax(m[k], u.kval(c[r][k]) + l);
             }
         }
+        // the workgroup's maximum of every column
+#pragma unroll
+        for (int k = 0; k < TC; ++k)
+            __hip_atomic_fetch_max(&S->cm[(k * WC + wc) * 64 + lane], order_key(m[k]),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < TC; ++k)
+            m[k] = shift_of(of_order_key(S->cm[(k * WC + wc) * 64 + lane]));
 #pragma unroll 1
         for (int r0 = 0; r0 < TR; r0 += RG) {
             T c[RG][TC];
@@ -415,15 +435,12 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
                 const double l = S->rl[wr * TR + r0 + r];
 #pragma unroll
                 for (int k = 0; k < TC; ++k)
-                    s[k] += U::term((u.kval(c[r][k]) + l) - shift_of(m[k]));
+                    s[k] += U::term((u.kval(c[r][k]) + l) - m[k]);
             }
         }
 #pragma unroll
-        for (int k = 0; k < TC; ++k) {
-            const int j = (k * WC + wc) * 64 + lane;
-            S->cm[wr * CW + j] = m[k];
-            S->cp[wr * CW + j] = s[k];
-        }
+        for (int k = 0; k < TC; ++k)
+            S->cp[wr * CW + (k * WC + wc) * 64 + lane] = s[k];
     }
     __syncthreads();
     const uint32_t tag = seq << 1;
@@ -432,41 +449,34 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     int late = 0;
     uint32_t unused = 0;
     // this workgroup's (max, sum) of column j
-    auto local_pair = [&](int j, float &m, double &s) {
-        m = S->cm[j];
-#pragma unroll
-        for (int w = 1; w < WR; ++w)
-            m = fmaxf(m, S->cm[w * CW + j]);
-        const double sh = shift_of(m);
+    auto local_pair = [&](int j, double &m, double &s) {
+        m = of_order_key(S->cm[j]);
         s = 0.0;
-#pragma unroll 1
-        for (int w = 0; w < WR; ++w) {
-            const double sw = (double)S->cp[w * CW + j];
-            if (sw != 0.0)
-                s += sw * U::expm(shift_of(S->cm[w * CW + j]) - sh);
-        }
+#pragma unroll
+        for (int w = 0; w < WR; ++w)
+            s += (double)S->cp[w * CW + j];
     };
     if (G > 1) {
         for (int j = t; j < M; j += F::NT) {
-            float m;
-            double s;
+            double m, s;
             local_pair(j, m, s);
             uint64_t *p = pw + (size_t)J.g * XW * Mp + j;
-            put_word(p, __float_as_uint(m), tag);
+            const uint64_t qm = (uint64_t)__double_as_longlong(m);
+            put_word(p, (uint32_t)qm, tag);
+            put_word(p + Mp, (uint32_t)(qm >> 32), tag);
             if constexpr (PW == 1) {
-                put_word(p + Mp, __float_as_uint((float)s), tag);
+                put_word(p + 2 * (size_t)Mp, __float_as_uint((float)s), tag);
             } else {
                 const uint64_t q = (uint64_t)__double_as_longlong(s);
-                put_word(p + Mp, (uint32_t)q, tag);
-                put_word(p + 2 * (size_t)Mp, (uint32_t)(q >> 32), tag);
+                put_word(p + 2 * (size_t)Mp, (uint32_t)q, tag);
+                put_word(p + 3 * (size_t)Mp, (uint32_t)(q >> 32), tag);
             }
         }
     }
 #pragma unroll 1
     for (int jl = t; jl < J.cn; jl += F::NT) {
         const int j = J.j0 + jl;
-        float m = -INFINITY;
-        double s = 0.0;
+        double m = -INFINITY, s = 0.0;
         if (G == 1) {
             local_pair(j, m, s);
         } else {
@@ -475,14 +485,15 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
 #pragma unroll 1
             for (int q = 0; q < G; ++q) {
                 const uint64_t *p = pw + (size_t)q * XW * Mp + j;
-                const float mq = __uint_as_float(wait_word(p, tag, unused, late));
+                const uint32_t mlo = wait_word(p, tag, unused, late);
+                const double mq = pack_d(mlo, wait_word(p + Mp, tag, unused, late));
                 double sq;
-                const uint32_t lo = wait_word(p + Mp, tag, unused, late);
+                const uint32_t lo = wait_word(p + 2 * (size_t)Mp, tag, unused, late);
                 if constexpr (PW == 1)
                     sq = (double)__uint_as_float(lo);
                 else
-                    sq = pack_d(lo, wait_word(p + 2 * (size_t)Mp, tag, unused, late));
-                const float mn = fmaxf(m, mq);
+                    sq = pack_d(lo, wait_word(p + 3 * (size_t)Mp, tag, unused, late));
+                const double mn = fmax(m, mq);
                 const double sh = shift_of(mn);
                 s = (s != 0.0 ? s * U::expm(shift_of(m) - sh) : 0.0) +
                     (sq != 0.0 ? sq * U::expm(shift_of(mq) - sh) : 0.0);
@@ -967,7 +978,7 @@ sk_resident(const ResArgs A) {
                 };
                 uint32_t tag = 0;
                 // this exchange's slots; a word's byte offset in them fits 32
-                // bits (at most 256 workgroups x 2 words x 4096 columns x 8)
+                // bits (at most 256 workgroups x 4 words x 4096 columns x 8)
                 const char *pw = nullptr;
                 char *cw = nullptr;
                 const uint32_t prow = (uint32_t)(XW * Mp) * 8u;  // one workgroup's partials

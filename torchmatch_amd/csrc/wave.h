@@ -358,4 +358,23 @@ __device__ __forceinline__ float wave_max_all(float x) {
     a = row_swap32_pair(x, o);
     return fmaxf(a, o);
 }
+
+// The same in float64, on wave_sum_all_d's butterfly.
+__device__ __forceinline__ double wave_max_all_d(double x) {
+    x = fmax(x, dpp_full_d<kDppQuadXor1>(x));
+    x = fmax(x, dpp_full_d<kDppQuadXor2>(x));
+    x = fmax(x, dpp_full_d<kDppRowHalfMirror>(x));
+    x = fmax(x, dpp_full_d<kDppRowMirror>(x));
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    u32x2 lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)u, false, false);
+    u32x2 hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false,
+                                                false);
+    x = fmax(__longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])),
+             __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1])));
+    const uint64_t v = (uint64_t)__double_as_longlong(x);
+    lo = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+    return fmax(__longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])),
+                __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1])));
+}
 } // namespace tmamd
