@@ -158,6 +158,71 @@ def test_far_row_and_column(B, N, M, dtype, far, where, mode, device, monkeypatc
     assert err <= bound
 
 
+@pytest.mark.parametrize("mode", [None, "exact"])
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize(("B", "N", "M"), [(3, 64, 80), (1, 400, 300), (1, 300, 1200)])
+def test_unbalanced_large_costs(B, N, M, dtype, mode, device, monkeypatch):
+    """Costs far above rho: the plan's mass, and with it every multiplier, is
+    e^-(cost / 2 rho) or less, below any float, while the log plan is an ordinary
+    number.  A constant added to every cost; an isolated pair (a row and a
+    column far from all others and close to each other) and an isolated row;
+    two blocks whose masses differ by e^-150; a far column of finite costs.
+    Epsilon and rho are powers of two, the same in both types."""
+    if mode:
+        monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_RESIDENT", mode)
+    dt = getattr(torch, dtype)
+    base = workloads.sinkhorn_points(B, N, M, 8, seed=M).to(dt)
+    a, b = workloads.dirichlet(B, N, seed=1).to(dt), workloads.dirichlet(B, M, seed=2).to(dt)
+    cases = {f"offset {x}": base + x for x in (200.0, 500.0, 3000.0)}
+    c = base.clone()
+    c[:, 3, :] = c[:, :, 7] = 400.0
+    c[:, 3, 7] = 0.5
+    c[:, 9, :] = 700.0
+    cases["isolated"] = c
+    c = base + 300.0
+    c[:, : N // 2, : M // 2] -= 300.0
+    c[:, : N // 2, M // 2 :] = c[:, N // 2 :, : M // 2] = 9000.0
+    cases["blocks"] = c
+    c = base.clone()
+    c[:, :, 7] = 1e9
+    cases["far column"] = c
+    for name, cost in cases.items():
+        kw = {"rho": 1.0, "n_iter": 30 if name != "offset 500.0" else 100}
+        ref = sk.unbalanced_sinkhorn_plan(cost.double(), eps=0.125, a=a.double(), b=b.double(),
+                                          dtype=torch.float64, **kw)[0]
+        got = solve(cost.to(device), backend=Backend.UNBALANCED_SINKHORN, reg=0.125,
+                    a=a.to(device), b=b.to(device), **kw)
+        scale = 1.0 + ref[torch.isfinite(ref)].abs()
+        sk_parity.logp_err(got, ref)  # the same entries finite
+        err = ((got.cpu().double() - ref).abs()[torch.isfinite(ref)] / scale).max().item()
+        # float32: the parity bound, and the output's and K's rounding (2^-24 of
+        # an entry each); float64: a few roundings of the same size
+        bound = 1e-5 if dtype == "float32" else 64 * 2.0 ** -52
+        print(f"unbalanced {name} {(B, N, M)} {dtype} {mode}: {err:.2e}", flush=True)
+        assert err <= bound, (name, err)
+
+
+@pytest.mark.parametrize("rho", [None, 0.3])
+@pytest.mark.parametrize(("B", "N", "M"), [(2, 60, 90), (1, 400, 300)])
+def test_denormal_marginals(B, N, M, rho, device):
+    """Masses below float32's normal range: their multipliers' reciprocals are
+    not float32 numbers."""
+    cost = workloads.sinkhorn_points(B, N, M, 8, seed=N)
+    a, b = workloads.dirichlet(B, N, seed=6), workloads.dirichlet(B, M, seed=7)
+    a[:, 5], b[:, 11], b[:, 20] = 1e-40, 3e-39, 1e-44
+    kw = {"a": a.to(device), "b": b.to(device), "reg": 0.05, "n_iter": 20}
+    if rho is None:
+        ref = sk.log_sinkhorn_plan(cost, eps=0.05, n_iter=20, a=a, b=b, dtype=torch.float64)[0]
+        got = solve(cost.to(device), **kw)
+    else:
+        ref = sk.unbalanced_sinkhorn_plan(cost, eps=0.05, n_iter=20, rho=rho, a=a, b=b,
+                                          dtype=torch.float64)[0]
+        got = solve(cost.to(device), backend=Backend.UNBALANCED_SINKHORN, rho=rho, **kw)
+    err = sk_parity.logp_err(got, ref)
+    # log masses down to -101: one float32 rounding of that (4e-6) more
+    assert err <= sk_parity.ELEM_BOUND + 4e-6, err
+
+
 @pytest.mark.parametrize(("B", "N", "M"), [
     (1, 1810, 43), (51, 634, 42), (1, 2000, 17), (2, 700, 5), (1, 1500, 1), (1, 700, 100)])
 def test_fewer_workgroups_than_merge_groups(B, N, M, device):

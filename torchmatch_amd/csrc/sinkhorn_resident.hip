@@ -15,7 +15,7 @@ constexpr int kCus = 256;
 
 // Words of the exchange buffer a problem in flight needs.
 size_t xch_words(int G, int64_t Mp, bool f64) {
-    const size_t xw = f64 ? 4 : 3, bw = f64 ? 4 : 3;
+    const size_t xw = f64 ? 4 : 3, bw = 4;
     return 2 * ((size_t)G * xw + bw) * (size_t)Mp;
 }
 

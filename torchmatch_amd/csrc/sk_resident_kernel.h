@@ -15,7 +15,14 @@
 // are two matrix-vector products and no exponential:
 //     LSE_j(K_ij + log_v_j) = rl_i + log S_i     S_i = sum_j P_ij b_j
 //     LSE_i(K_ij + log_u_i) = c_j  + log T_j     T_j = sum_i P_ij a_i
-// and, balanced, a_i = mu_i / S_i, b_j = nu_j / T_j.  P is rounded to float32
+// and, balanced, a_i = mu_i / S_i, b_j = nu_j / T_j.  Unbalanced, the potentials
+// themselves are kept too (log_u and log_v in float64): they are damped, so a
+// multiplier is not near its marginal but as small as the plan's mass, which
+// large costs take out of any float's range.  A scale kappa common to the
+// problem is therefore taken out there, P = e^(K - rl - c + kappa), a =
+// e^(log_u + rl - kappa), b = e^(log_v + c - kappa) (0 for balanced solves): the
+// exact step sets it to the largest column's, so that the columns' and rows'
+// multipliers lie around 1 whatever the mass.  P is rounded to float32
 // once (relative 2^-24 per entry; the K of the streaming step is rounded to
 // float32 at |K| ~ 40, about 2^-19), lane sums are float32 of TC or TR terms,
 // sums across lanes and waves and the multipliers are float64.  The float32
@@ -30,8 +37,11 @@
 // 2^20, so what is lost is below 2^-32 of a sum.  A step outside the window
 // (and the first) is done exactly from the cost, with the maximum taken out
 // of every sum, the reference's logsumexp, and P is rebuilt around the new
-// potentials.  A row or column whose LSE is not finite keeps its potential, as
-// the reference's isfinite rule has it.  When epsilon changes, P is rebuilt
+// potentials.  Unbalanced multipliers have no lower bound (what underflows is
+// held as a potential, and contributes less than 2^-150 P to a sum), so a P
+// with an entry above 2^60 (both its row and its column carry less than 2^-60
+// of the mass) is refused there.  A row or column whose LSE is not finite keeps
+// its potential, as the reference's isfinite rule has it.  When epsilon changes, P is rebuilt
 // from the cost around the current potentials and the step goes on.
 //
 // Several workgroups per problem.  Each holds `rows` whole rows, so the row
@@ -61,6 +71,11 @@ namespace tmamd {
 namespace {
 
 constexpr double kSumLo = 0x1p-60, kSumHi = 0x1p60, kMulHi = 0x1p20;
+// unbalanced P above this is refused (kPHi<double>: doubles underflow 2^-1022)
+template <typename T> constexpr T kPHi = (T)0x1p60;
+template <> constexpr double kPHi<double> = 0x1p900;
+// float multipliers below this carry no rounding (their reciprocal overflows)
+constexpr float kCarryLo = 0x1p-120f;
 // a wait longer than this (100 MHz ticks) ends the solve with NaN potentials
 constexpr uint64_t kWaitTicks = 400000000ull;
 
@@ -179,6 +194,8 @@ template <int N, typename Fn> __device__ __forceinline__ void unroll(Fn &&f) {
     unroll_seq(f, std::make_integer_sequence<int, N>{});
 }
 
+__device__ __forceinline__ float max_t(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double max_t(double a, double b) { return fmax(a, b); }
 __device__ __forceinline__ float readlane_t(float x, int lane) { return readlane_f(x, lane); }
 __device__ __forceinline__ double readlane_t(double x, int lane) { return readlane_d(x, lane); }
 
@@ -244,7 +261,7 @@ template <typename T, int NW_, int LC_, int WC_, int TC_, int TR_, bool SOLO_> s
     static constexpr int KC = SOLO ? NK : 1;               // owned columns per thread
     static constexpr int PW = Unit<T>::kPartWords;  // words of a column partial
     static constexpr int XW = PW + 2;               // words of an exact partial (max, sum)
-    static constexpr int BW = PW + 2;               // words of an exact broadcast (c, b)
+    static constexpr int BW = 4;                    // words of an exact broadcast (c, log_v)
     static_assert(RW <= 64 && RW % 4 == 0, "one row per lane");
     static __device__ __forceinline__ int col(int k, int wc, int lane) {
         return (k * WC + wc) * LC + (lane & (LC - 1));
@@ -258,9 +275,13 @@ template <typename F> struct Shared {
     double rl[F::R];               // row references (exact step: log_u)
     double xs[F::NT];              // split column sums
     double bd[F::KC * F::NT];        // owned columns: multiplier and marginal
-    double nu[F::KC * F::NT];        // (unbalanced: in log units)
+    double nu[F::KC * F::NT];        // (unbalanced: log_v and log marginal)
+    double kappa;                  // the scale taken out (unbalanced)
     double rm[F::WC * F::R];       // exact step: row maxima
-    uint64_t cm[F::CW];            // exact step: column maxima (order_key)
+    union {                        // exact step:
+        double lv[F::CW];          // log_v of all columns, which it starts from
+        uint64_t cm[F::CW];        // then the column maxima (order_key)
+    };
     T b[F::CW];
     T cp[F::WR * F::CW];           // column sums of each row wave
     float eb[F::KC * F::NT];
@@ -325,14 +346,12 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     const int wr = wid / WC, wc = wid % WC;
     const int M = J.M, Mp = J.Mp, G = J.G;
     const U u(eps);
-    for (int j = t; j < CW; j += F::NT)
-        S->cm[j] = order_key(-INFINITY);
     {
         double lvk[TC];
 #pragma unroll
         for (int k = 0; k < TC; ++k) {
             const int j = (k * WC + wc) * 64 + lane;
-            lvk[k] = U::logm((double)S->b[j]) - S->c[j];
+            lvk[k] = S->lv[j];
         }
 #pragma unroll 1
         for (int r0 = 0; r0 < TR; r0 += RG) {
@@ -364,6 +383,8 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
         }
     }
     __syncthreads();
+    for (int j = t; j < CW; j += F::NT)
+        S->cm[j] = order_key(-INFINITY);
     double lse = 0.0;
     const int rho = lane_row(lane), row = wr * TR + rho;
     const bool has = rho < TR && row < J.nrow;
@@ -501,50 +522,101 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
             }
         }
         const double l = U::logm(s) + shift_of(m);
-        double lv = U::logm(S->bd[jl]) - S->c[j];
+        double lv = J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[j];
         const bool dc = !isfinite(l);
         if (!dc) {
             const double d = U::of_nat(J.lnu[j]) - l;
             lv = J.unbal ? damp * d : d;
         }
-        const double cr = !dc ? l : isfinite(lv) ? -lv : 0.0;
-        const double b = U::expm(lv + cr);
-        S->bd[jl] = b;
+        const double cr = !dc ? l : NAN;  // (set below once kappa is known)
         S->eb[jl] = 0.f;
         S->dead[jl] = dc;
-        S->c[j] = cr;
-        S->b[j] = (T)b;
         if (G > 1 && !J.direct) {
             const uint64_t q = (uint64_t)__double_as_longlong(cr);
             put_word(cw + j, (uint32_t)q, tag);
             put_word(cw + Mp + j, (uint32_t)(q >> 32), tag);
-            if constexpr (PW == 1) {
-                put_word(cw + 2 * (size_t)Mp + j, __float_as_uint((float)b), tag);
-            } else {
-                const uint64_t qb = (uint64_t)__double_as_longlong(b);
-                put_word(cw + 2 * (size_t)Mp + j, (uint32_t)qb, tag);
-                put_word(cw + 3 * (size_t)Mp + j, (uint32_t)(qb >> 32), tag);
-            }
+            const uint64_t ql = (uint64_t)__double_as_longlong(lv);
+            put_word(cw + 2 * (size_t)Mp + j, (uint32_t)ql, tag);
+            put_word(cw + 3 * (size_t)Mp + j, (uint32_t)(ql >> 32), tag);
+        } else {
+            S->c[j] = cr;
+            S->lv[j] = lv;
         }
     }
+    __syncthreads();
     if (G > 1 && !J.direct) {
-        __syncthreads();
         for (int j = t; j < M; j += F::NT) {
             const uint32_t lo = wait_word(cw + j, tag, unused, late);
             S->c[j] = pack_d(lo, wait_word(cw + Mp + j, tag, unused, late));
-            const uint32_t b0 = wait_word(cw + 2 * (size_t)Mp + j, tag, unused, late);
-            if constexpr (PW == 1)
-                S->b[j] = __uint_as_float(b0);
-            else
-                S->b[j] = pack_d(b0, wait_word(cw + 3 * (size_t)Mp + j, tag, unused, late));
+            const uint32_t l0 = wait_word(cw + 2 * (size_t)Mp + j, tag, unused, late);
+            S->lv[j] = pack_d(l0, wait_word(cw + 3 * (size_t)Mp + j, tag, unused, late));
         }
     }
+    // kappa, the same in every workgroup (each has all columns, a thread the
+    // columns it stored); then the multipliers around it
+    double kap = 0.0;
+    if (J.unbal) {
+        double m = -INFINITY;
+        for (int j = t; j < M; j += F::NT)
+            m = fmax(m, S->lv[j] + S->c[j]);  // (NaN, a dead column, drops out)
+        m = wave_max_all_d(m);
+        if (lane == 0)
+            S->xs[wid] = m;
+        __syncthreads();
+        for (int w = 0; w < F::NW; ++w)
+            m = fmax(m, S->xs[w]);
+        kap = isfinite(m) ? m : 0.0;
+    }
+    for (int j = t; j < M; j += F::NT) {
+        const double lv = S->lv[j];
+        double c = S->c[j];
+        if (isnan(c))
+            S->c[j] = c = isfinite(lv) ? kap - lv : 0.0;
+        S->b[j] = (T)U::expm(lv + c - kap);
+    }
+    if (t == 0)
+        S->kappa = kap;
     if (late)
         S->abort = 1;
+    __syncthreads();
+    for (int jl = t; jl < J.cn; jl += F::NT) {
+        const int j = J.j0 + jl;
+        S->bd[jl] = J.unbal ? S->lv[j] : U::expm(S->lv[j] + S->c[j]);
+    }
     if (has) {
-        W.rl = !W.dead ? lse : isfinite(W.lu) ? -W.lu : 0.0;
-        W.a = U::expm(W.lu + W.rl);
+        W.rl = !W.dead ? lse : isfinite(W.lu) ? kap - W.lu : 0.0;
+        W.a = U::expm(W.lu + W.rl - kap);
         W.ea = 0.f;
+    }
+    __syncthreads();
+}
+
+// A step was refused: log_v of the last accepted one, for the exact step.
+template <typename F>
+__device__ __noinline__ void send_log_v(SharedP<F> S, const Job &J, uint32_t seq) {
+    using U = Unit<typename F::Type>;
+    const uint32_t tag = seq << 1;
+    uint64_t *cw = J.cast + (size_t)(seq & 1) * F::BW * J.Mp;
+    for (int jl = (int)threadIdx.x; jl < J.cn; jl += F::NT) {
+        const int j = J.j0 + jl;
+        const double lv = J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[j];
+        if (J.direct) {
+            S->lv[j] = lv;
+        } else {
+            const uint64_t q = (uint64_t)__double_as_longlong(lv);
+            put_word(cw + j, (uint32_t)q, tag);
+            put_word(cw + J.Mp + j, (uint32_t)(q >> 32), tag);
+        }
+    }
+    if (!J.direct) {
+        int late = 0;
+        uint32_t unused = 0;
+        for (int j = (int)threadIdx.x; j < J.M; j += F::NT) {
+            const uint32_t lo = wait_word(cw + j, tag, unused, late);
+            S->lv[j] = pack_d(lo, wait_word(cw + J.Mp + j, tag, unused, late));
+        }
+        if (late)
+            S->abort = 1;
     }
     __syncthreads();
 }
@@ -563,7 +635,7 @@ __device__ __noinline__ void recentre(SharedP<F> S, const Job &J, Row &W) {
         S->b[j] = (T)ldexp(b, -e);
         S->c[j] -= U::of_exp2(e);
         const int jl = j - J.j0;
-        if (jl >= 0 && jl < J.cn)
+        if (jl >= 0 && jl < J.cn && !J.unbal)
             S->bd[jl] = ldexp(S->bd[jl], -e);
     }
     // rows the lane does not have hold a = 0
@@ -590,9 +662,12 @@ __device__ __noinline__ void start_problem(SharedP<F> S, const Job &J, Row &W, c
     for (int j = t; j < F::CW; j += F::NT) {
         S->c[j] = j < J.M ? 0.0 : INFINITY;  // columns past M: P = 0, b = 0
         S->b[j] = j < J.M ? (T)1 : (T)0;
+        S->lv[j] = 0.0;
     }
+    if (t == 0)
+        S->kappa = 0.0;
     for (int jl = t; jl < F::KC * F::NT; jl += F::NT) {
-        S->bd[jl] = 1.0;
+        S->bd[jl] = J.unbal ? 0.0 : 1.0;
         S->eb[jl] = 0.f;
         S->dead[jl] = 0;
         const double l = jl < J.cn ? U::of_nat(J.lnu[J.j0 + jl]) : -INFINITY;
@@ -622,7 +697,8 @@ __device__ __noinline__ void finish_problem(SharedP<F> S, const Job &J, Row &W,
     if (!J.direct || J.g == 0) {
         for (int jl = t; jl < J.cn; jl += F::NT) {
             const double x =
-                failed ? NAN : U::to_nat(U::logm(S->bd[jl]) - S->c[J.j0 + jl]);
+                failed ? NAN
+                       : U::to_nat(J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[J.j0 + jl]);
             log_v[J.j0 + jl] = (T)x;
             if (lv64 != nullptr)
                 lv64[J.j0 + jl] = x;
@@ -708,8 +784,9 @@ sk_resident(const ResArgs A) {
             const double damp = unbal ? 1.0 / (1.0 + eps / A.rho) : 1.0;
 
             // ---- P around the references ---------------------------------------
+            const double kap = unbal ? readlane_d(S.kappa, 0) : 0.0;
             if (!trial && wc == 0 && rho < RW)
-                S.rl[lrow] = has ? W.rl : INFINITY;
+                S.rl[lrow] = has ? W.rl - kap : INFINITY;
             if (t < 2) {
                 S.flag_row[t] = 0;
                 S.flag_all[t] = 0;
@@ -801,7 +878,7 @@ sk_resident(const ResArgs A) {
                         W.rl = __builtin_isfinite(mine) ? u.kval((T)mine) : 0.0;
                     }
                     if (wc == 0 && rho < RW)
-                        S.rl[lrow] = has ? W.rl : INFINITY;
+                        S.rl[lrow] = has ? W.rl : INFINITY;  // (kappa is 0)
                     __syncthreads();
                 }
                 double ck[TC];
@@ -819,11 +896,21 @@ sk_resident(const ResArgs A) {
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                if (unbal) {
+                    T top = (T)0;
+#pragma unroll
+                    for (int r = 0; r < TR; ++r)
+#pragma unroll
+                        for (int k = 0; k < TC; ++k)
+                            top = max_t(top, v[r][k]);
+                    if (ballot(top > kPHi<T>) != 0 && lane == 0)
+                        S.flag_row[0] = 1;  // refuses the first step
+                }
             }
             Row L = W;  // W is in memory (it is passed to the calls above)
-            // the thread's owned columns t + kc * 512: multiplier, its carried
-            // rounding, the marginal (balanced linear, else in log units), the
-            // reference
+            // the thread's owned columns t + kc * NT: multiplier (unbalanced:
+            // log_v), the rounding its float32 copy carries, the marginal
+            // (balanced linear, else in log units), the reference
             double cb[KC], cnu[KC], cref[KC];
             float ceb[KC];
             bool cdead[KC];
@@ -898,7 +985,7 @@ sk_resident(const ResArgs A) {
                         a_new = L.mu * U::recip(rsum);
                     } else {
                         lu_new = damp * (L.lmu - (U::log_fast(rsum) + L.rl));
-                        a_new = U::exp_fast(lu_new + L.rl);
+                        a_new = U::exp_fast(lu_new + L.rl - kap);
                     }
                     const bool ok = L.dead ? rsum == 0.0
                                            : rsum >= kSumLo && rsum <= kSumHi && a_new <= mul_hi;
@@ -909,7 +996,7 @@ sk_resident(const ResArgs A) {
                     if constexpr (PW == 1) {
                         const double x = fma(a_new, (double)L.ea, a_new);
                         ah = (float)x;
-                        if (ah != 0.f)
+                        if (ah > kCarryLo)
                             ea_new = (float)(x - (double)ah) * __builtin_amdgcn_rcpf(ah);
                     } else {
                         ah = a_new;
@@ -1102,23 +1189,24 @@ sk_resident(const ResArgs A) {
                     }
                     double b;
                     if (!unbal) {
-                        b = cnu[kc] * U::recip(s);
+                        b = cdead[kc] ? cb[kc] : cnu[kc] * U::recip(s);
+                        b_new[kc] = b;
                     } else {
                         const double c = cref[kc];
-                        b = U::exp_fast(damp * (cnu[kc] - (U::log_fast(s) + c)) + c);
+                        const double lv =
+                            cdead[kc] ? cb[kc] : damp * (cnu[kc] - (U::log_fast(s) + c));
+                        b = U::exp_fast(lv + c - kap);
+                        b_new[kc] = lv;
                     }
                     const bool ok = cdead[kc] ? s == 0.0
                                               : s >= kSumLo && s <= kSumHi && b <= mul_hi;
-                    if (cdead[kc])
-                        b = cb[kc];
                     bad |= ok ? 0u : 1u;
-                    b_new[kc] = b;
                     eb_new[kc] = 0.f;
                     T h;
                     if constexpr (PW == 1) {
                         const double x = fma(b, (double)ceb[kc], b);
                         h = (float)x;
-                        if (h != 0.f)
+                        if (h > kCarryLo)
                             eb_new[kc] = (float)(x - (double)h) * __builtin_amdgcn_rcpf(h);
                     } else {
                         h = b;
@@ -1185,35 +1273,6 @@ sk_resident(const ResArgs A) {
                     S.abort = 1;
                 __syncthreads();
                 if (S.flag_all[fp] | S.abort) {
-                    // refused: the multipliers of the last accepted step again
-                    if (!direct) {
-                        ++seq;
-                        tag = seq << 1;
-                        cw = reinterpret_cast<char *>(cast + (size_t)(seq & 1) * BW * Mp);
-                    }
-#pragma unroll
-                    for (int kc = 0; kc < KC; ++kc) {
-                        const int jl = t + kc * F::NT;
-                        if (jl >= cn)
-                            break;
-                        S.b[j0 + jl] = (T)cb[kc];
-                        if (!direct) {
-                            uint64_t *p = reinterpret_cast<uint64_t *>(cw + (uint32_t)(j0 + jl) * 8u);
-                            if constexpr (PW == 1) {
-                                put_word(p, __float_as_uint((float)cb[kc]), tag);
-                            } else {
-                                const uint64_t x = (uint64_t)__double_as_longlong(cb[kc]);
-                                put_word(p, (uint32_t)x, tag);
-                                put_word(p + Mp, (uint32_t)(x >> 32), tag);
-                            }
-                        }
-                    }
-                    if (!direct) {
-                        late = 0;
-                        gather_b();
-                        if (late)
-                            S.abort = 1;
-                    }
                     start = kExact;
                     break;
                 }
@@ -1243,6 +1302,11 @@ sk_resident(const ResArgs A) {
                 S.eb[t + kc * F::NT] = ceb[kc];
             }
             __syncthreads();
+            if (start == kExact) {  // refused
+                if (!direct)
+                    ++seq;
+                send_log_v<F>(SP, J, seq);
+            }
         }
         finish_problem<F>(SP, J, W, static_cast<T *>(A.log_u) + prob * A.N + i0,
                           A.lu64 ? A.lu64 + prob * A.N + i0 : nullptr,
