@@ -821,7 +821,10 @@ sk_resident(const ResArgs A) {
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if (keep != nullptr) {
-                    constexpr int KR = TR < 4 ? TR : 4;  // rows in flight
+                    // rows in flight: 16 mask bytes a lane or so (four rows of 16
+                    // spilled half of P: the start of (16, 2048, 2048) 512 us
+                    // against 640)
+                    constexpr int KR = TC >= 12 ? 1 : TC >= 6 ? 2 : TR < 4 ? TR : 4;
 #pragma unroll
                     for (int r0 = 0; r0 < TR; r0 += KR) {
                         uint8_t kp[KR][TC];
@@ -926,6 +929,13 @@ sk_resident(const ResArgs A) {
 
             // ---- steps from P until epsilon changes or one is refused ----------
             for (int fp = 0;; fp ^= 1) {
+                // the thread's columns, anew each step: kept over the loop, their
+                // addresses do not fit the registers beside 128 matrix entries
+                // and come back from scratch one by one, each waited for together
+                // with the stores before it (us per step with them and without:
+                // (16, 2048, 2048) 32.6, 23.6; (1, 4096, 4096) 12.1, 9.6)
+                int tj = t;
+                asm volatile("" : "+v"(tj));
                 double rsum = 0.0;  // the lane's row
                 {
                     T bk[TC];
@@ -1137,7 +1147,7 @@ sk_resident(const ResArgs A) {
                     char *mine = const_cast<char *>(pw) + (uint32_t)g * prow;
 #pragma unroll
                     for (int kc = 0; kc < F::NK; ++kc) {
-                        const int j = t + kc * F::NT;
+                        const int j = tj + kc * F::NT;
                         if (j < M) {
                             const double s = local_sum(j);
                             uint64_t *p = reinterpret_cast<uint64_t *>(mine + (uint32_t)j * 8u);
@@ -1173,7 +1183,7 @@ sk_resident(const ResArgs A) {
                 float eb_new[KC];
 #pragma unroll
                 for (int kc = 0; kc < KC; ++kc) {
-                    const int jl = t + kc * F::NT;
+                    const int jl = tj + kc * F::NT;
                     if (jl >= cn)
                         break;
                     const int j = j0 + jl;
@@ -1237,7 +1247,7 @@ sk_resident(const ResArgs A) {
 #pragma unroll
                             for (int p = 0; p < PW; ++p)
                                 w[kc][p] = get_word(reinterpret_cast<const uint64_t *>(
-                                    cw + (uint32_t)(min(t + kc * F::NT, M - 1) + p * Mp) * 8u));
+                                    cw + (uint32_t)(min(tj + kc * F::NT, M - 1) + p * Mp) * 8u));
 #pragma unroll
                         for (int kc = 0; kc < NK; ++kc)
 #pragma unroll
@@ -1253,13 +1263,12 @@ sk_resident(const ResArgs A) {
 #pragma unroll
                     for (int kc = 0; kc < NK; ++kc) {
                         bad |= (uint32_t)(w[kc][0] >> 32);
-                        const int j = t + kc * F::NT;
+                        const int j = tj + kc * F::NT;
                         if (j < M) {
                             if constexpr (PW == 1)
-                                S.b[t + kc * F::NT] = __uint_as_float((uint32_t)w[kc][0]);
+                                S.b[j] = __uint_as_float((uint32_t)w[kc][0]);
                             else
-                                S.b[t + kc * F::NT] =
-                                    pack_d((uint32_t)w[kc][0], (uint32_t)w[kc][PW - 1]);
+                                S.b[j] = pack_d((uint32_t)w[kc][0], (uint32_t)w[kc][PW - 1]);
                         }
                     }
                 };
