@@ -31,10 +31,12 @@
 // converged multiplier does not drive the potentials' neutral mode
 // (log_u + c, log_v - c) step after step.
 //
-// When that is exact enough.  P underflows below 2^-149 and its absolute error
-// there is below 2^-126 max(a, b) per entry; a step is accepted only while
-// every S_i and T_j lies in [2^-60, 2^60] and every multiplier is at most
-// 2^20, so what is lost is below 2^-32 of a sum.  A step outside the window
+// When that is exact enough.  P is denormal below 2^-126, off by at most 2^-150
+// an entry; a step is accepted only while every S_i and T_j lies in [2^-60,
+// 2^60] and every multiplier its sums use is at most 2^40, so that what is lost
+// is below 2^-150 2^40 2^17 (rows a problem may have) 2^60 = 2^-33 of a sum.
+// (The column multipliers of the first step may go to 2^60: P is rebuilt around
+// them before they are used.)  A step outside the window
 // (and the first) is done exactly from the cost, with the maximum taken out
 // of every sum, the reference's logsumexp, and P is rebuilt around the new
 // potentials.  Unbalanced multipliers have no lower bound (what underflows is
@@ -70,7 +72,7 @@
 namespace tmamd {
 namespace {
 
-constexpr double kSumLo = 0x1p-60, kSumHi = 0x1p60, kMulHi = 0x1p20;
+constexpr double kSumLo = 0x1p-60, kSumHi = 0x1p60, kMulHi = 0x1p40;
 // unbalanced P above this is refused (kPHi<double>: doubles underflow 2^-1022)
 template <typename T> constexpr T kPHi = (T)0x1p60;
 template <> constexpr double kPHi<double> = 0x1p900;
@@ -221,21 +223,30 @@ struct Waiter {
     }
 };
 
-// Payload of the word at p once its tag is `tag` (bit 0 of the tag is the
-// sender's bad flag, OR-ed into `bad`).
-__device__ __forceinline__ uint32_t wait_word(const uint64_t *p, uint32_t tag, uint32_t &bad,
-                                              int &timed_out) {
-    uint64_t w = get_word(p);
+// Payloads of the words p(0) ... p(N - 1) once all carry `tag`, all in flight
+// at a time.
+template <int N, typename P>
+__device__ __forceinline__ void wait_words(P &&p, uint32_t tag, uint32_t (&x)[N], int &late) {
+    uint64_t w[N];
     Waiter wt;
-    while (((uint32_t)(w >> 32) | 1u) != (tag | 1u)) {
-        if (!wt.more()) {
-            timed_out = 1;
+    for (;;) {
+        uint32_t diff = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            w[i] = get_word(p(i));
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            diff |= (uint32_t)(w[i] >> 32) ^ tag;
+        if (diff == 0)
+            break;
+        if (late != 0 || !wt.more()) {
+            late = 1;
             break;
         }
-        w = get_word(p);
     }
-    bad |= (uint32_t)(w >> 32) & 1u;
-    return (uint32_t)w;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        x[i] = (uint32_t)w[i];
 }
 
 // One workgroup's share of a problem, R rows of up to CW columns, in one of
@@ -274,6 +285,7 @@ template <typename F> struct Shared {
     double rs[F::WC * F::R];       // row sums of each column wave
     double rl[F::R];               // row references (exact step: log_u)
     double xs[F::NT];              // split column sums
+    double xm[F::SOLO ? 1 : F::NT];  // exact step: split column maxima
     double bd[F::KC * F::NT];        // owned columns: multiplier and marginal
     double nu[F::KC * F::NT];        // (unbalanced: log_v and log marginal)
     double kappa;                  // the scale taken out (unbalanced)
@@ -310,7 +322,7 @@ struct Job {
     const uint8_t *keep;
     const double *lnu;
     uint64_t *part, *cast;
-    int M, Mp, G, g, nrow, j0, cn, direct, unbal;
+    int M, Mp, G, g, nrow, j0, cn, cnp, direct, unbal;
 };
 
 template <typename F, typename T>
@@ -318,14 +330,26 @@ __device__ __forceinline__ void load_rows(const Job &J, int row, int wc, int lan
                                           T (&c)[F::ETC]) {
     const T *C = static_cast<const T *>(J.C);
     const int64_t base = (int64_t)min(row, J.nrow - 1) * J.M;
+    // every load goes out unconditionally (in bounds), then what is not there
+    // becomes +inf: behind a condition each load is waited for
+    uint8_t kp[F::ETC];
+#pragma unroll
+    for (int k = 0; k < F::ETC; ++k)
+        c[k] = C[base + min((k * F::WC + wc) * 64 + lane, J.M - 1)];
+    if (J.keep != nullptr) {
+#pragma unroll
+        for (int k = 0; k < F::ETC; ++k)
+            kp[k] = J.keep[base + min((k * F::WC + wc) * 64 + lane, J.M - 1)];
+    } else {
+#pragma unroll
+        for (int k = 0; k < F::ETC; ++k)
+            kp[k] = 1;
+    }
 #pragma unroll
     for (int k = 0; k < F::ETC; ++k) {
         const int j = (k * F::WC + wc) * 64 + lane;
-        const int64_t o = base + min(j, J.M - 1);
-        bool ok = row < J.nrow && j < J.M;
-        if (J.keep != nullptr)
-            ok = ok && J.keep[o] != 0;
-        c[k] = ok ? C[o] : (T)INFINITY;
+        const bool ok = (row < J.nrow) & (j < J.M) & (kp[k] != 0);
+        c[k] = ok ? c[k] : (T)INFINITY;
     }
 }
 
@@ -468,7 +492,6 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     uint64_t *pw = J.part + (size_t)(seq & 1) * G * XW * Mp;
     uint64_t *cw = J.cast + (size_t)(seq & 1) * BW * Mp;
     int late = 0;
-    uint32_t unused = 0;
     // this workgroup's (max, sum) of column j
     auto local_pair = [&](int j, double &m, double &s) {
         m = of_order_key(S->cm[j]);
@@ -494,33 +517,57 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
             }
         }
     }
+    double gm = -INFINITY, gs = 0.0;  // column t of the owned ones, all workgroups
+    if constexpr (!F::SOLO) {
+        // thread groups share a column's partials as in the step, each in
+        // workgroup order, then the groups' results in theirs: the same in
+        // every workgroup that merges this column.  Four partials in flight:
+        // one by one, and with load_rows' loads behind conditions, this step
+        // took 200 us for four problems of 2048 x 2048 at a time; 50 now, most
+        // of it float64 arithmetic (four rows in flight: no faster)
+        auto add = [](double &m, double &s, double mq, double sq) {
+            const double mn = fmax(m, mq), sh = shift_of(mn);
+            s = (s != 0.0 ? s * U::expm(shift_of(m) - sh) : 0.0) +
+                (sq != 0.0 ? sq * U::expm(shift_of(mq) - sh) : 0.0);
+            m = mn;
+        };
+        const int split = F::NT / J.cnp, sp = t / J.cnp, jl = t % J.cnp;
+        double m = -INFINITY, s = 0.0;
+        if (jl < J.cn) {
+            const uint64_t *p = pw + J.j0 + jl;
+#pragma unroll 1
+            for (int q0 = sp; q0 < G; q0 += 4 * split) {
+                uint32_t x[4 * XW];
+                wait_words<4 * XW>(
+                    [&](int i) {
+                        const int q = min(q0 + i / XW * split, G - 1);
+                        return p + ((size_t)q * XW + i % XW) * Mp;
+                    },
+                    tag, x, late);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t *xi = x + i * XW;
+                    const double sq =
+                        PW == 1 ? (double)__uint_as_float(xi[2]) : pack_d(xi[2], xi[XW - 1]);
+                    if (q0 + i * split < G)
+                        add(m, s, pack_d(xi[0], xi[1]), sq);
+                }
+            }
+        }
+        S->xm[t] = m;
+        S->xs[t] = s;
+        __syncthreads();
+        if (t < J.cn) {
+            for (int k = 0; k < min(split, G); ++k)
+                add(gm, gs, S->xm[k * J.cnp + t], S->xs[k * J.cnp + t]);
+        }
+    }
 #pragma unroll 1
     for (int jl = t; jl < J.cn; jl += F::NT) {
         const int j = J.j0 + jl;
-        double m = -INFINITY, s = 0.0;
-        if (G == 1) {
+        double m = gm, s = gs;
+        if (F::SOLO)
             local_pair(j, m, s);
-        } else {
-            // running merge in workgroup order, the same in every workgroup
-            // that merges this column
-#pragma unroll 1
-            for (int q = 0; q < G; ++q) {
-                const uint64_t *p = pw + (size_t)q * XW * Mp + j;
-                const uint32_t mlo = wait_word(p, tag, unused, late);
-                const double mq = pack_d(mlo, wait_word(p + Mp, tag, unused, late));
-                double sq;
-                const uint32_t lo = wait_word(p + 2 * (size_t)Mp, tag, unused, late);
-                if constexpr (PW == 1)
-                    sq = (double)__uint_as_float(lo);
-                else
-                    sq = pack_d(lo, wait_word(p + 3 * (size_t)Mp, tag, unused, late));
-                const double mn = fmax(m, mq);
-                const double sh = shift_of(mn);
-                s = (s != 0.0 ? s * U::expm(shift_of(m) - sh) : 0.0) +
-                    (sq != 0.0 ? sq * U::expm(shift_of(mq) - sh) : 0.0);
-                m = mn;
-            }
-        }
         const double l = U::logm(s) + shift_of(m);
         double lv = J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[j];
         const bool dc = !isfinite(l);
@@ -545,11 +592,18 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
     }
     __syncthreads();
     if (G > 1 && !J.direct) {
-        for (int j = t; j < M; j += F::NT) {
-            const uint32_t lo = wait_word(cw + j, tag, unused, late);
-            S->c[j] = pack_d(lo, wait_word(cw + Mp + j, tag, unused, late));
-            const uint32_t l0 = wait_word(cw + 2 * (size_t)Mp + j, tag, unused, late);
-            S->lv[j] = pack_d(l0, wait_word(cw + 3 * (size_t)Mp + j, tag, unused, late));
+#pragma unroll 1
+        for (int j = t; j < M; j += 2 * F::NT) {
+            const int j1 = min(j + F::NT, M - 1);  // (the last column twice at most)
+            uint32_t x[8];
+            wait_words<8>([&](int i) { return cw + (i & 3) * (size_t)Mp + (i < 4 ? j : j1); },
+                          tag, x, late);
+            S->c[j] = pack_d(x[0], x[1]);
+            S->lv[j] = pack_d(x[2], x[3]);
+            if (j + F::NT < M) {
+                S->c[j1] = pack_d(x[4], x[5]);
+                S->lv[j1] = pack_d(x[6], x[7]);
+            }
         }
     }
     // kappa, the same in every workgroup (each has all columns, a thread the
@@ -610,10 +664,10 @@ __device__ __noinline__ void send_log_v(SharedP<F> S, const Job &J, uint32_t seq
     }
     if (!J.direct) {
         int late = 0;
-        uint32_t unused = 0;
         for (int j = (int)threadIdx.x; j < J.M; j += F::NT) {
-            const uint32_t lo = wait_word(cw + j, tag, unused, late);
-            S->lv[j] = pack_d(lo, wait_word(cw + J.Mp + j, tag, unused, late));
+            uint32_t x[2];
+            wait_words<2>([&](int i) { return cw + (size_t)i * J.Mp + j; }, tag, x, late);
+            S->lv[j] = pack_d(x[0], x[1]);
         }
         if (late)
             S->abort = 1;
@@ -755,7 +809,8 @@ sk_resident(const ResArgs A) {
     for (int64_t prob = cluster; prob < A.B; prob += A.clusters) {
         const int64_t off = (prob * A.N + i0) * (int64_t)M;
         const Job J{static_cast<const T *>(A.cost) + off, A.keep ? A.keep + off : nullptr,
-                    A.lnu + prob * M, part, cast, M, Mp, G, g, nrow, j0, cn, direct, unbal};
+                    A.lnu + prob * M, part, cast, M, Mp, G, g, nrow, j0, cn, cnp, direct,
+                    unbal};
         Row W;
         start_problem<F>(SP, J, W, A.lmu + prob * A.N + i0);
 
@@ -933,9 +988,12 @@ sk_resident(const ResArgs A) {
                 // addresses do not fit the registers beside 128 matrix entries
                 // and come back from scratch one by one, each waited for together
                 // with the stores before it (us per step with them and without:
-                // (16, 2048, 2048) 32.6, 23.6; (1, 4096, 4096) 12.1, 9.6)
+                // (16, 2048, 2048) 32.6, 23.6; (1, 4096, 4096) 12.1, 9.6; float64
+                // (2, 300, 200) 3.4, 3.1).  A small tile of one workgroup has room
+                // for them ((64, 64, 80): 0.89 a step kept, 0.90 not)
                 int tj = t;
-                asm volatile("" : "+v"(tj));
+                if constexpr (!SOLO || TC * TR >= 96)
+                    asm volatile("" : "+v"(tj));
                 double rsum = 0.0;  // the lane's row
                 {
                     T bk[TC];
@@ -998,7 +1056,7 @@ sk_resident(const ResArgs A) {
                         a_new = U::exp_fast(lu_new + L.rl - kap);
                     }
                     const bool ok = L.dead ? rsum == 0.0
-                                           : rsum >= kSumLo && rsum <= kSumHi && a_new <= mul_hi;
+                                           : rsum >= kSumLo && rsum <= kSumHi && a_new <= kMulHi;
                     if (L.dead || !has) {
                         a_new = L.a;
                         lu_new = L.lu;
