@@ -12,12 +12,16 @@ namespace tmamd {
 namespace {
 
 constexpr int kCus = 256;
+constexpr uint32_t kMaxPolls = 4u << 20;  // of 1 us or more each
 
 // Words of the exchange buffer a problem in flight needs.
 size_t xch_words(int G, int64_t Mp, bool f64) {
     const size_t xw = f64 ? 4 : 3, bw = 4;
     return 2 * ((size_t)G * xw + bw) * (size_t)Mp;
 }
+
+// Bytes of the problems' marks, behind it.
+size_t mark_bytes(int64_t B) { return ((size_t)B * sizeof(uint32_t) + 15) / 16 * 16; }
 
 const Tile &tile_of(int k, bool f64) {
     if (f64)
@@ -80,7 +84,9 @@ SkResidentPlan sk_resident_plan(int64_t B, int64_t N, int64_t M, bool f64) {
             best.direct = direct ? 1 : 0;
             const int64_t Mp = (M + 15) / 16 * 16;
             best.xch_bytes =
-                G == 1 ? 0 : sizeof(uint64_t) * xch_words((int)G, Mp, f64) * (size_t)clusters;
+                G == 1 ? 0
+                       : sizeof(uint64_t) * xch_words((int)G, Mp, f64) * (size_t)clusters +
+                             mark_bytes(B);
         }
     }
     // the streaming step: launches and merge, then the matrix at 7 TB/s, read
@@ -139,6 +145,12 @@ int sk_resident_launch(const SkResidentPlan &plan, const SkResidentIo &io, int64
     // "exact": every step from the cost (how the tests reach that path)
     const char *env = getenv("TORCHMATCH_AMD_SINKHORN_RESIDENT");
     A.exact_only = env != nullptr && strcmp(env, "exact") == 0;
+    // "late": no wait at all, every shared problem is given up
+    A.max_polls = env != nullptr && strcmp(env, "late") == 0 ? 0 : kMaxPolls;
+    A.given_up = nullptr;
+    if (plan.G > 1)
+        A.given_up = reinterpret_cast<uint32_t *>(static_cast<char *>(io.xch) + plan.xch_bytes -
+                                                  mark_bytes(B));
     // exchange numbers stay below 2^31: at most three per step
     const int64_t rounds = (B + plan.clusters - 1) / plan.clusters;
     if (plan.G > 1 && rounds * 3 * ((int64_t)n_iter + 1) >= (1ll << 30))

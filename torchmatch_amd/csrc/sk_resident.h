@@ -18,7 +18,7 @@ struct SkResidentPlan {
     int clusters;  // problems in flight
     int rows;      // rows per workgroup
     int direct;    // every workgroup merges every column (else column owners)
-    size_t xch_bytes;  // exchange buffer (0 when G == 1)
+    size_t xch_bytes;  // exchange buffer and the problems' marks (0 when G == 1)
 };
 
 SkResidentPlan sk_resident_plan(int64_t B, int64_t N, int64_t M, bool f64);
@@ -31,6 +31,8 @@ struct ResArgs {
     void *log_u, *log_v;
     double *lu64, *lv64;
     uint64_t *xch;
+    uint32_t *given_up;      // a mark per problem
+    uint32_t max_polls;      // longest wait for another workgroup
     int64_t B;
     int N, M, Mp;            // Mp: columns rounded up to 16 (exchange rows)
     int G, clusters, rows, direct, cpo;

@@ -55,8 +55,12 @@
 // columns every workgroup merges all of them (one hop, `direct`); else
 // workgroup g owns a range of columns, merges it and sends its multipliers to
 // the others (two hops).  Such a grid is launched cooperatively, which
-// guarantees that all its workgroups are resident, and every wait is bounded
-// in time.
+// guarantees that all its workgroups become resident; when the last of them does
+// is up to whatever else runs on the device.  Every wait is bounded all the
+// same, in polls (time in which a wave does not run itself does not count): a
+// workgroup whose wait has lasted 4 million of them, some seconds, gives its
+// problem up, and whoever is the first to do so marks it for the others and
+// solves it alone from the cost (redo_problem).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -78,8 +82,6 @@ template <typename T> constexpr T kPHi = (T)0x1p60;
 template <> constexpr double kPHi<double> = 0x1p900;
 // float multipliers below this carry no rounding (their reciprocal overflows)
 constexpr float kCarryLo = 0x1p-120f;
-// a wait longer than this (100 MHz ticks) ends the solve with NaN potentials
-constexpr uint64_t kWaitTicks = 400000000ull;
 
 // The log unit of each type: base 2 on the native v_exp_f32 for float costs,
 // natural with the library's exp / log for double costs.
@@ -209,26 +211,40 @@ __device__ __forceinline__ uint64_t get_word(const uint64_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A bounded wait: false once the launch has waited longer than kWaitTicks.
+// A bounded wait for workgroups of the same problem: false once it has lasted
+// ResArgs::max_polls (asked every 1024 polls), or one of them has given the
+// problem up.  `args` fetches the arguments there and then: a polling loop keeps
+// the count alone (limit, clock and mark in its registers cost 0.1 us a step of
+// (1, 1024, 1024)).
 struct Waiter {
-    uint32_t polls = 0;
-    uint64_t start = 0;
-    __device__ bool more() {
+    uint32_t polls;
+    __device__ explicit Waiter(uint32_t first) : polls(first) {}
+    template <typename Args> __device__ bool more(Args &&args, int64_t prob) {
         if ((++polls & 1023u) != 0)
             return true;
-        const uint64_t now = wall_clock64();
-        if (start == 0)
-            start = now;
-        return now - start < kWaitTicks;
+        const ResArgs *A = args();
+        return polls < A->max_polls && __hip_atomic_load(A->given_up + prob, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT) == 0;
     }
 };
+// The first count: with a limit of 0 the first poll is the last.
+__device__ __forceinline__ uint32_t first_poll(uint32_t max_polls) {
+    return max_polls == 0 ? 1023u : 0u;
+}
+// The kernel's arguments where they are (in the kernel itself only).
+__device__ __forceinline__ const ResArgs *res_args() {
+    const ResArgs *A = (const ResArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(A));  // not read ahead of need
+    return A;
+}
 
 // Payloads of the words p(0) ... p(N - 1) once all carry `tag`, all in flight
 // at a time.
 template <int N, typename P>
-__device__ __forceinline__ void wait_words(P &&p, uint32_t tag, uint32_t (&x)[N], int &late) {
+__device__ __forceinline__ void wait_words(const ResArgs *A, int64_t prob, P &&p, uint32_t tag,
+                                           uint32_t (&x)[N], int &late) {
     uint64_t w[N];
-    Waiter wt;
+    Waiter wt(first_poll(A->max_polls));
     for (;;) {
         uint32_t diff = 0;
 #pragma unroll
@@ -239,7 +255,7 @@ __device__ __forceinline__ void wait_words(P &&p, uint32_t tag, uint32_t (&x)[N]
             diff |= (uint32_t)(w[i] >> 32) ^ tag;
         if (diff == 0)
             break;
-        if (late != 0 || !wt.more()) {
+        if (late != 0 || !wt.more([A] { return A; }, prob)) {
             late = 1;
             break;
         }
@@ -322,6 +338,8 @@ struct Job {
     const uint8_t *keep;
     const double *lnu;
     uint64_t *part, *cast;
+    const ResArgs *args;
+    int64_t prob;
     int M, Mp, G, g, nrow, j0, cn, cnp, direct, unbal;
 };
 
@@ -539,6 +557,7 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
             for (int q0 = sp; q0 < G; q0 += 4 * split) {
                 uint32_t x[4 * XW];
                 wait_words<4 * XW>(
+                    J.args, J.prob,
                     [&](int i) {
                         const int q = min(q0 + i / XW * split, G - 1);
                         return p + ((size_t)q * XW + i % XW) * Mp;
@@ -596,8 +615,9 @@ __device__ __noinline__ void exact_step(SharedP<F> S, const Job &J, Row &W, doub
         for (int j = t; j < M; j += 2 * F::NT) {
             const int j1 = min(j + F::NT, M - 1);  // (the last column twice at most)
             uint32_t x[8];
-            wait_words<8>([&](int i) { return cw + (i & 3) * (size_t)Mp + (i < 4 ? j : j1); },
-                          tag, x, late);
+            wait_words<8>(
+                J.args, J.prob,
+                [&](int i) { return cw + (i & 3) * (size_t)Mp + (i < 4 ? j : j1); }, tag, x, late);
             S->c[j] = pack_d(x[0], x[1]);
             S->lv[j] = pack_d(x[2], x[3]);
             if (j + F::NT < M) {
@@ -666,7 +686,8 @@ __device__ __noinline__ void send_log_v(SharedP<F> S, const Job &J, uint32_t seq
         int late = 0;
         for (int j = (int)threadIdx.x; j < J.M; j += F::NT) {
             uint32_t x[2];
-            wait_words<2>([&](int i) { return cw + (size_t)i * J.Mp + j; }, tag, x, late);
+            wait_words<2>(
+                J.args, J.prob, [&](int i) { return cw + (size_t)i * J.Mp + j; }, tag, x, late);
             S->lv[j] = pack_d(x[0], x[1]);
         }
         if (late)
@@ -730,7 +751,68 @@ __device__ __noinline__ void start_problem(SharedP<F> S, const Job &J, Row &W, c
     __syncthreads();
 }
 
-// The potentials of a finished problem (NaN when a wait ran out).
+// A problem that was given up, by one workgroup: every half-step from the cost
+// with the maximum taken out, the potentials (in log units until the end) in
+// global memory, no other workgroup needed.
+template <typename T> __device__ __noinline__ void redo_problem(const ResArgs *A, int64_t p) {
+    using U = Unit<T>;
+    const int t = (int)threadIdx.x, nt = (int)blockDim.x, lane = lane_id();
+    const int N = A->N, M = A->M;
+    const T *C = static_cast<const T *>(A->cost) + p * N * (int64_t)M;
+    const uint8_t *keep = A->keep != nullptr ? A->keep + p * N * (int64_t)M : nullptr;
+    double *lu = (A->lu64 != nullptr ? A->lu64 : static_cast<double *>(A->log_u)) + p * N;
+    double *lv = (A->lv64 != nullptr ? A->lv64 : static_cast<double *>(A->log_v)) + p * M;
+    for (int i = t; i < N; i += nt)
+        lu[i] = 0.0;
+    for (int j = t; j < M; j += nt)
+        lv[j] = 0.0;
+    __syncthreads();
+    int seg = 0;
+    for (int it = 0; it < A->n_iter; ++it) {
+        if (it == A->seg_end[seg])
+            ++seg;
+        const U u(A->eps[seg]);
+        const double damp = A->rho > 0.0 ? 1.0 / (1.0 + A->eps[seg] / A->rho) : 1.0;
+        auto value = [&](int64_t o) {
+            return u.kval(keep == nullptr || keep[o] != 0 ? C[o] : (T)INFINITY);
+        };
+        for (int i = t >> 6; i < N; i += nt / 64) {  // a wave per row
+            const int64_t o = (int64_t)i * M;
+            double m = -INFINITY, s = 0.0;
+            for (int j = lane; j < M; j += 64)
+                m = fmax(m, value(o + j) + lv[j]);
+            m = shift_of(wave_max_all_d(m));
+            for (int j = lane; j < M; j += 64)
+                s += (double)U::term(value(o + j) + lv[j] - m);
+            const double lse = U::logm(wave_sum_all_d(s)) + m;
+            if (lane == 0 && isfinite(lse))
+                lu[i] = damp * (U::of_nat(A->lmu[p * N + i]) - lse);
+        }
+        __syncthreads();
+        for (int j = t; j < M; j += nt) {  // a thread per column
+            double m = -INFINITY, s = 0.0;
+            for (int i = 0; i < N; ++i)
+                m = fmax(m, value((int64_t)i * M + j) + lu[i]);
+            m = shift_of(m);
+            for (int i = 0; i < N; ++i)
+                s += (double)U::term(value((int64_t)i * M + j) + lu[i] - m);
+            const double lse = U::logm(s) + m;
+            if (isfinite(lse))
+                lv[j] = damp * (U::of_nat(A->lnu[p * M + j]) - lse);
+        }
+        __syncthreads();
+    }
+    for (int i = t; i < N; i += nt)
+        static_cast<T *>(A->log_u)[p * N + i] = (T)(lu[i] = U::to_nat(lu[i]));
+    for (int j = t; j < M; j += nt)
+        static_cast<T *>(A->log_v)[p * M + j] = (T)(lv[j] = U::to_nat(lv[j]));
+}
+
+// The potentials of a finished problem.  One that this workgroup gave up (and all
+// that follow it: its exchanges are no longer those of the others) it solves
+// alone, unless another has.  A workgroup that came through the last exchange all
+// the same writes its results too, before or after: every value is that of a
+// whole solve either way.
 template <typename F>
 __device__ __noinline__ void finish_problem(SharedP<F> S, const Job &J, Row &W,
                                             typename F::Type *log_u, double *lu64,
@@ -738,12 +820,24 @@ __device__ __noinline__ void finish_problem(SharedP<F> S, const Job &J, Row &W,
     using T = typename F::Type;
     using U = Unit<T>;
     const int t = (int)threadIdx.x;
-    const bool failed = S->abort != 0;
+    if (S->abort != 0) {
+        if constexpr (!F::SOLO) {
+            if (t == 0)
+                S->flag_row[0] =
+                    __hip_atomic_exchange(J.args->given_up + J.prob, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT) == 0;
+            __syncthreads();
+            if (S->flag_row[0] != 0)
+                redo_problem<T>(J.args, J.prob);
+            __syncthreads();
+        }
+        return;
+    }
     const int rho = lane_row(lane_id()), row = (t >> 6) / F::WC * F::RW + rho;
     if ((t >> 6) % F::WC == 0 && rho < F::RW && row < J.nrow) {
         if (W.derived && !W.dead && !J.unbal)
             W.lu = U::logm(W.a) - W.rl;
-        const double x = failed ? NAN : U::to_nat(W.lu);
+        const double x = U::to_nat(W.lu);
         log_u[row] = (T)x;
         if (lu64 != nullptr)
             lu64[row] = x;
@@ -751,8 +845,7 @@ __device__ __noinline__ void finish_problem(SharedP<F> S, const Job &J, Row &W,
     if (!J.direct || J.g == 0) {
         for (int jl = t; jl < J.cn; jl += F::NT) {
             const double x =
-                failed ? NAN
-                       : U::to_nat(J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[J.j0 + jl]);
+                U::to_nat(J.unbal ? S->bd[jl] : U::logm(S->bd[jl]) - S->c[J.j0 + jl]);
             log_v[J.j0 + jl] = (T)x;
             if (lv64 != nullptr)
                 lv64[J.j0 + jl] = x;
@@ -801,6 +894,7 @@ sk_resident(const ResArgs A) {
     const int rho = lane_row(lane), lrow = wr * RW + rho;  // the lane's row
     const bool has = rho < RW && lrow < nrow;
     const bool odd = lane & 1, odd2 = lane & 2;
+    const uint32_t poll0 = SOLO ? 0 : first_poll(A.max_polls);
     uint32_t seq = 0;
     if (t == 0)
         S.abort = 0;
@@ -809,8 +903,8 @@ sk_resident(const ResArgs A) {
     for (int64_t prob = cluster; prob < A.B; prob += A.clusters) {
         const int64_t off = (prob * A.N + i0) * (int64_t)M;
         const Job J{static_cast<const T *>(A.cost) + off, A.keep ? A.keep + off : nullptr,
-                    A.lnu + prob * M, part, cast, M, Mp, G, g, nrow, j0, cn, cnp, direct,
-                    unbal};
+                    A.lnu + prob * M, part, cast, res_args(), prob, M, Mp, G, g, nrow, j0, cn,
+                    cnp, direct, unbal};
         Row W;
         start_problem<F>(SP, J, W, A.lmu + prob * A.N + i0);
 
@@ -1150,7 +1244,7 @@ sk_resident(const ResArgs A) {
                     double acc = 0.0;
                     for (int u0 = 0; u0 < per; u0 += N) {
                         uint64_t w[N][PW];
-                        Waiter wt;
+                        Waiter wt(poll0);
                         for (;;) {
                             uint32_t diff = 0;
 #pragma unroll
@@ -1171,7 +1265,7 @@ sk_resident(const ResArgs A) {
                                 bad |= diff;
                                 break;
                             }
-                            if (!wt.more()) {
+                            if (!wt.more(res_args, prob)) {
                                 late = 1;
                                 break;
                             }
@@ -1297,7 +1391,7 @@ sk_resident(const ResArgs A) {
                 auto gather_b = [&]() {
                     constexpr int NK = F::NK;
                     uint64_t w[NK][PW];
-                    Waiter wt;
+                    Waiter wt(poll0);
                     for (;;) {
                         uint32_t diff = 0;
 #pragma unroll
@@ -1313,7 +1407,7 @@ sk_resident(const ResArgs A) {
                                 diff |= (uint32_t)(w[kc][p] >> 32) ^ tag;
                         if (diff <= 1u)
                             break;
-                        if (!wt.more()) {
+                        if (!wt.more(res_args, prob)) {
                             late = 1;
                             break;
                         }
@@ -1369,7 +1463,7 @@ sk_resident(const ResArgs A) {
                 S.eb[t + kc * F::NT] = ceb[kc];
             }
             __syncthreads();
-            if (start == kExact) {  // refused
+            if (start == kExact && !S.abort) {  // refused
                 if (!direct)
                     ++seq;
                 send_log_v<F>(SP, J, seq);
