@@ -323,6 +323,7 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
 constexpr int kPrepWaves = 4;                                // waves per prepare block
 constexpr int kPrepRowsPerWave = 8;                          // rows a wave keeps in flight
 constexpr int kPrepRows = kPrepWaves * kPrepRowsPerWave;     // rows per block and group
+constexpr int kHeldWord = 2;  // of the statistics: the epsilon of K, behind flags and maximum
 constexpr uint32_t kFlagNan = TM_SK_FLAG_NAN, kFlagNegInf = TM_SK_FLAG_NEG_INF;
 constexpr uint32_t kFlagANeg = TM_SK_FLAG_A_NEG, kFlagBNeg = TM_SK_FLAG_B_NEG;
 
@@ -345,10 +346,21 @@ __device__ __forceinline__ float k_of(float c, float e, double s2) {
     return s2 != 0.0 ? (float)((double)c * s2) : -c / e;
 }
 
+// `held` (may be null): the epsilon of K as it is in the workspace.  With
+// `unless_held` nothing is done where it is eps already; else it becomes eps.
 template <bool MASK>
 __global__ void __launch_bounds__(kMapBlock)
 sk_log_kernel(const float *__restrict__ C, const uint8_t *__restrict__ keep,
-              float *__restrict__ K, int64_t n, float eps, double s2, int vec) {
+              float *__restrict__ K, int64_t n, float eps, double s2, int vec, float *held,
+              int unless_held) {
+    if (held != nullptr) {
+        if (unless_held) {
+            if (*held == eps)
+                return;
+        } else if (blockIdx.x == 0 && threadIdx.x == 0) {
+            *held = eps;
+        }
+    }
     const int64_t stride = (int64_t)gridDim.x * kMapBlock;
     const int64_t n4 = vec ? n / 4 : 0;
     const float4 *c4 = reinterpret_cast<const float4 *>(C);
@@ -406,17 +418,18 @@ sk_fill64(double *__restrict__ y, int64_t n, double value) {
         y[k] = value;
 }
 
-// Start state of sk_prepare: every row and column flagged all-+inf, stats 0.
+// Start state of sk_prepare: every row and column flagged all-+inf, stats 0, K
+// about to hold k_eps (0: none).
 __global__ void __launch_bounds__(kMapBlock)
 sk_reset_flags(uint8_t *__restrict__ inf_row, int64_t n_row, uint8_t *__restrict__ inf_col,
-               int64_t n_col, uint32_t *__restrict__ stats) {
+               int64_t n_col, uint32_t *__restrict__ stats, float k_eps) {
     const int64_t k = (int64_t)blockIdx.x * kMapBlock + threadIdx.x;
     if (k < n_row)
         inf_row[k] = 1;
     if (k < n_col)
         inf_col[k] = 1;
-    if (k < 2)
-        stats[k] = 0;
+    if (k <= kHeldWord)
+        stats[k] = k == kHeldWord ? __float_as_uint(k_eps) : 0;
 }
 
 // One pass over the cost C (B, N, M) and the optional keep mask:
@@ -1663,17 +1676,17 @@ bool shape_supported(const SinkhornLayout &L) {
 // K for one epsilon: the reference's -C'/e (two-sweep step), or with `base2`
 // the fused step's -C'*log2(e)/e.
 int launch_log_kernel(const float *cost, const uint8_t *keep, float *K, int64_t nK, float e,
-                      bool base2, hipStream_t stream) {
+                      bool base2, float *held, int unless_held, hipStream_t stream) {
     const double s2 = base2 ? -kLog2eD / (double)e : 0.0;
     const int vec = ((uintptr_t)cost % 16) == 0 && ((uintptr_t)K % 16) == 0 &&
                     ((uintptr_t)keep % 4) == 0;
     const dim3 grid(grid_for(nK / 4 + 1, kMapBlock, 8192));
     if (keep != nullptr)
         TM_LAUNCH(sk_log_kernel<true>, grid, dim3(kMapBlock), 0, stream, cost, keep, K, nK, e,
-                  s2, vec);
+                  s2, vec, held, unless_held);
     else
         TM_LAUNCH(sk_log_kernel<false>, grid, dim3(kMapBlock), 0, stream, cost, keep, K, nK, e,
-                  s2, vec);
+                  s2, vec, held, unless_held);
     return TM_OK;
 }
 
@@ -1946,15 +1959,15 @@ extern "C" int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *ke
     uint8_t *inf_col = reinterpret_cast<uint8_t *>(ws + L.off_infcol);
     uint32_t *stats = reinterpret_cast<uint32_t *>(ws + L.off_stats);
 
-    const int64_t n_flags = B * N > B * M ? B * N : B * M;
+    if (resident_ok(L, form, workspace, stream))
+        k_eps = 0.f;  // the resident solve reads the cost, not K
+    int64_t n_flags = B * N > B * M ? B * N : B * M;
+    n_flags = n_flags > kHeldWord ? n_flags : kHeldWord + 1;
     TM_LAUNCH(sk_reset_flags, dim3(grid_for(n_flags, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
-              stream, inf_row, B * N, inf_col, B * M, stats);
-    const bool resident = resident_ok(L, form, workspace, stream);
+              stream, inf_row, B * N, inf_col, B * M, stats, k_eps);
     const bool state64 = L.fused != kFzNone || L.res.cfg >= 0;
     double *mu64 = state64 ? reinterpret_cast<double *>(ws + L.off_mu64) : nullptr;
     double *nu64 = state64 ? reinterpret_cast<double *>(ws + L.off_nu64) : nullptr;
-    if (resident)
-        k_eps = 0.f;  // the resident solve reads the cost, not K
     TM_LAUNCH(sk_log_marginal, dim3(grid_for(B * N, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
               stream, a, log_mu, mu64, B * N, stats, kFlagANeg);
     TM_LAUNCH(sk_log_marginal, dim3(grid_for(B * M, kMapBlock, 1 << 30)), dim3(kMapBlock), 0,
@@ -2085,8 +2098,14 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
         if (rc != TM_ERR_UNSUPPORTED_SHAPE)
             return rc;
     }
-    if (resident_form(L, form))
-        k_eps = 0.f;  // the preparation pass left K to this call
+    // The preparation pass leaves K to this call when it expects it to run
+    // resident (not under capture, say); which it did, the workspace knows.
+    float *held = L.res.cfg >= 0 ? reinterpret_cast<float *>(ws + L.off_stats) + kHeldWord : nullptr;
+    if (resident_form(L, form) && k_eps > 0.f) {
+        const int rc = launch_log_kernel(cost, keep, K, nK, k_eps, fused, held, 1, stream);
+        if (rc != TM_OK)
+            return rc;
+    }
 
     TM_LAUNCH(sk_fill, dim3(grid_for(B * N, kMapBlock, 1 << 30)), dim3(kMapBlock), 0, stream,
               log_u, B * N, 0.f);
@@ -2123,7 +2142,7 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
             const float e = (float)eps_sched[s0];
             bool exact0 = s0 == 0;
             if (e != cur_eps) {
-                const int rc = launch_log_kernel(cost, keep, K, nK, e, true, stream);
+                const int rc = launch_log_kernel(cost, keep, K, nK, e, true, held, 0, stream);
                 if (rc != TM_OK)
                     return rc;
                 cur_eps = e;
@@ -2170,7 +2189,7 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
     for (int32_t s = 0; s < n_iter && !fused; ++s) {
         const float e = (float)eps_sched[s];
         if (e != cur_eps) {  // K holds -C / e for the step's epsilon
-            const int rc = launch_log_kernel(cost, keep, K, nK, e, false, stream);
+            const int rc = launch_log_kernel(cost, keep, K, nK, e, false, held, 0, stream);
             if (rc != TM_OK)
                 return rc;
             cur_eps = e;
