@@ -253,6 +253,7 @@ def test_batch_groups_match_oracle(groups, device, monkeypatch):
     r32, r64 = _balanced_refs(cost, 0.05, 30, a, b, scaling=0.5)
     args = (cost.to(device),)
     kw = dict(reg=0.05, n_iter=30, a=a.to(device), b=b.to(device), scaling=0.5)
+    monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_FUSED", "1")  # not the resident solve
     monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_GROUPS", groups)
     plan = solve(*args, **kw)
     monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_GROUPS", "1")

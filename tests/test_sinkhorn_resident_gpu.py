@@ -308,3 +308,22 @@ def test_streaming_groups_same_bits(B, N, M, device, monkeypatch):
         plans.append(solve(cost, **args))
     assert torch.equal(plans[0], plans[1]) and torch.equal(plans[0], plans[2])
     assert sk_parity.logp_err(plans[0], resident.cpu()) <= sk_parity.ELEM_BOUND
+
+
+def test_streaming_steps_still_match_oracle(device, monkeypatch):
+    """What other files hold to the oracle through calls that now run resident,
+    once more on the streaming steps."""
+    import test_sinkhorn_f64_gpu as f64
+    import test_sinkhorn_fullsize_gpu as full
+    import test_sinkhorn_gpu as f32
+
+    monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_RESIDENT", "0")
+    f64.test_unbalanced_f64_matches_oracle(device)
+    f64.test_f64_scaling_and_mask(device)
+    f32.test_step_shapes_match_oracle(None, (2, 150, 1500), device, monkeypatch)
+    f32.test_unbalanced_matches_oracle(1, 500, 300, 0.02, 100, 1.0, device)
+    f32.test_forbidden_cells_rows_and_columns(device)
+    case = full.INDEX["c4"]
+    cost, a, b = full._inputs(case)
+    full._check("C4 streaming", case, *full._run_device(case, cost, a, b, device), cost,
+                full._fixture(case))

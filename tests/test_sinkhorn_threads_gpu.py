@@ -7,7 +7,9 @@ streams the library owns, one set per device.  Two host threads call
 on its own torch stream with its own problem and workspace, many times in a
 row, so their fork / launch / join segments overlap in time.  Every result
 must equal, bit for bit, the same solve run alone with one group
-(TORCHMATCH_AMD_SINKHORN_GROUPS=1: every launch on the caller's stream).
+(TORCHMATCH_AMD_SINKHORN_GROUPS=1: every launch on the caller's stream).  The
+same once more without a step named: both problems are then solved in
+cooperative launches from the two streams.
 """
 
 from __future__ import annotations
@@ -59,7 +61,10 @@ class _Problem:
         return out
 
 
-def test_two_threads_two_streams_match_serial(device, monkeypatch):
+@pytest.mark.parametrize("step", ["fused", "resident"])
+def test_two_threads_two_streams_match_serial(step, device, monkeypatch):
+    if step == "fused":
+        monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_FUSED", "1")
     probs = [
         _Problem(4, 300, 1024, 0.05, 40, 0.0, seed=51, device=device),
         _Problem(3, 200, 2048, 0.02, 40, 1.0, seed=61, device=device),
@@ -91,7 +96,7 @@ def test_two_threads_two_streams_match_serial(device, monkeypatch):
             results[k].append(p.result(s))
 
     threads = [threading.Thread(target=worker, args=(k,)) for k in range(2)]
-    print("two threads, two streams, default batch groups", flush=True)
+    print(f"two threads, two streams, {step}, default batch groups", flush=True)
     for t in threads:
         t.start()
     for t in threads:
