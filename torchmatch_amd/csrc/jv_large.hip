@@ -97,13 +97,21 @@ __device__ __forceinline__ void load_row_raw(const CostView &C, int i, float (&r
         raw[e] = src[min(e * 64 + lane, C.M - 1)];
 }
 
+constexpr int kNotFinite = 0x207;  // NaN, -inf, +inf (v_cmp_class)
+
 // The padded-tile view of a raw cost: +inf -> sentinel, columns >= M -> 0.  In
 // bit operations: as selects it compiles to two branches per value (a row of
-// eight chunks then took 1500 cycles in scan_group).
+// eight chunks then took 1500 cycles in scan_group).  With up to four chunks a
+// lane a class compare and one select are the faster way to the sentinel
+// ((32, 200, 200) uniform 3.61 ms against 3.63), with more they are not ((4, 900,
+// 900) points 24.7 ms against 25.0).
+template <int NC>
 __device__ __forceinline__ float fix_cost(const CostView &C, float raw, int j) {
     const uint32_t u = __float_as_uint(raw), s = __float_as_uint(C.sentinel);
-    const uint32_t inf = (uint32_t)((int)(0x7f7fffffu - (u & 0x7fffffffu)) >> 31);
     const uint32_t in = (uint32_t)((j - C.M) >> 31);
+    if constexpr (NC <= 4)
+        return __uint_as_float((__builtin_amdgcn_classf(raw, kNotFinite) ? s : u) & in);
+    const uint32_t inf = (uint32_t)((int)(0x7f7fffffu - (u & 0x7fffffffu)) >> 31);
     return __uint_as_float(((u & ~inf) | (s & inf)) & in);
 }
 
@@ -116,7 +124,7 @@ __device__ __forceinline__ void load_row(const CostView &C, int i, float (&cr)[N
         load_row_raw<NC>(C, i, raw);
 #pragma unroll
         for (int e = 0; e < NC; ++e)
-            cr[e] = fix_cost(C, raw[e], e * 64 + lane);
+            cr[e] = fix_cost<NC>(C, raw[e], e * 64 + lane);
     } else {
 #pragma unroll
         for (int e = 0; e < NC; ++e)
@@ -621,7 +629,7 @@ __device__ __forceinline__ int scan_group(LDS &L, const CostView &C, int K, int 
         const int iq = L.y[jq];
         const float level = L.d[jq];
         float cq = C.src[(int64_t)min(iq, C.N - 1) * C.M + min(jq, C.M - 1)];
-        cq = iq < C.N ? fix_cost(C, cq, jq) : 0.f;
+        cq = iq < C.N ? fix_cost<NC>(C, cq, jq) : 0.f;
         const float h = cq - L.v[jq] - level;
         const int n = min(64, hi - done);
         float raw[D][NC];
@@ -1029,7 +1037,7 @@ __device__ __forceinline__ bool large_solve(const int K, const int E, LDS &L, co
 #pragma unroll
                 for (int e = 0; e < NC; ++e) {
                     const int j = e * 64 + lane;
-                    const float cv = fix_cost(C, c[q][e], j);
+                    const float cv = fix_cost<NC>(C, c[q][e], j);
                     if (i + q < rows_real && e < E && j < K && cv < vmin[e]) {
                         vmin[e] = cv;
                         ymin[e] = i + q;
@@ -1411,6 +1419,7 @@ __device__ __forceinline__ bool large_solve(const int K, const int E, LDS &L, co
     // serve (it ran out) or a real row takes the paths below.
     int *const run_list = reinterpret_cast<int *>(L.rbuf);
     int run_pos = 0, run_n = 0;
+    int group_skip = 0, group_back = 1;  // see scan_group's call
     for (int f = 0; f < n_free; ++f) {
         int start = uniform_i(L.fr[f]);
         if (start >= C.N && run_pos < run_n) {
@@ -1606,9 +1615,16 @@ __device__ __forceinline__ bool large_solve(const int K, const int E, LDS &L, co
             // scan_dense
             int slo = lo, shi = hi;
             bool early = false;
-            if (shi - slo >= kGroupScan) {
+            if (shi - slo >= kGroupScan && (NC > 2 || --group_skip < 0)) {
                 slo = scan_group<NC>(L, C, K, slo, shi, final_j);
                 early = final_j >= 0;
+                // Handed back: the problem's groups bring many joins.  Up to 128
+                // columns the set-up then costs more than it saves, and the next
+                // ones, up to four, are taken position by position at once ((32,
+                // 100, 100) of eight values 229 us without this, 224 with)
+                const bool back = slo != shi && !early;
+                group_skip = back ? group_back : 0;
+                group_back = back ? min(2 * group_back, 4) : 1;
             }
             while (slo != shi && !early) {
                 const int q = slo++;
@@ -1636,10 +1652,10 @@ __device__ __forceinline__ bool large_solve(const int K, const int E, LDS &L, co
 #pragma unroll
                     for (int e = 0; e < NC; ++e)
                         cg[e] = srow[min(jg[e], C.M - 1)];
-                    cq = fix_cost(C, cq, jq);
+                    cq = fix_cost<NC>(C, cq, jq);
 #pragma unroll
                     for (int e = 0; e < NC; ++e)
-                        cg[e] = fix_cost(C, cg[e], jg[e]);
+                        cg[e] = fix_cost<NC>(C, cg[e], jg[e]);
                 } else {
 #pragma unroll
                     for (int e = 0; e < NC; ++e)
@@ -1761,7 +1777,7 @@ jv_solve_large_kernel(const float *__restrict__ costs, int64_t B, int N, int M,
         // compact outside the wave path's range: the lane-serial transcription
         if (lane == 0) {
             auto cost = [C](int i, int j) {
-                return (i >= C.N || j >= C.M) ? 0.f : fix_cost(C, C.src[(int64_t)i * C.M + j], j);
+                return (i >= C.N || j >= C.M) ? 0.f : fix_cost<NC>(C, C.src[(int64_t)i * C.M + j], j);
             };
             L.ev[0] = compact_serial((uint32_t)K, cost, L.x, L.y, L.fr, L.pred, L.cols, L.v,
                                      L.d) ? 1 : 0;
