@@ -11,6 +11,7 @@ the 1e-5 the parity tests use.
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -254,6 +255,43 @@ def test_given_up(B, N, M, dtype, rho, device, monkeypatch):
         err = sk_parity.logp_err(solve(cost.to(device, dt), **kw), ref)
         print(f"given up {(B, N, M)} {dtype} rho {rho}: {err:.2e}", flush=True)
         assert err <= (sk_parity.ELEM_BOUND if dtype == "float32" else 2e-13)
+
+
+@pytest.mark.skipif(np.finfo(np.longdouble).nmant < 63, reason="needs an 80-bit long double")
+@pytest.mark.parametrize(("N", "M", "eps", "n_iter", "rho"), [
+    (300, 200, 0.05, 100, None), (64, 300, 0.1, 100, None), (300, 200, 0.05, 100, 1.0),
+    (120, 90, 0.02, 60, 0.5)])
+def test_float64_plan_is_no_further_from_80_bits(N, M, eps, n_iter, rho, device, monkeypatch):
+    """A float64 resident plan against the same recurrence in 80 bits, and the
+    streaming steps' plan: the resident one is no further off (2-norm; one
+    rounding of every entry is about 6e-17 of it)."""
+    cost = workloads.sinkhorn_points(1, N, M, 8, seed=N + 1).double()
+    a, b = (workloads.dirichlet(1, k, seed=s).double() for k, s in ((N, 1), (M, 2)))
+    L = np.longdouble
+    K = (-(cost[0].numpy() / eps)).astype(L)  # K as float64 has it, on both sides
+    la, lb = np.log(a[0].numpy().astype(L)), np.log(b[0].numpy().astype(L))
+    lu, lv = np.zeros(N, L), np.zeros(M, L)
+    damp = L(1.0 if rho is None else 1.0 / (1.0 + eps / rho))
+
+    def lse(x, axis):
+        m = x.max(axis)
+        return np.log(np.exp(x - np.expand_dims(m, axis)).sum(axis)) + m
+
+    for _ in range(n_iter):
+        lu = damp * (la - lse(K + lv[None, :], 1))
+        lv = damp * (lb - lse(K + lu[:, None], 0))
+    true = lu[:, None] + K + lv[None, :]
+    kw = {"a": a.to(device), "b": b.to(device), "reg": eps, "n_iter": n_iter}
+    if rho is not None:
+        kw |= {"backend": Backend.UNBALANCED_SINKHORN, "rho": rho}
+    err = []
+    for mode in (None, "0"):
+        if mode:
+            monkeypatch.setenv("TORCHMATCH_AMD_SINKHORN_RESIDENT", mode)
+        d = solve(cost.to(device), **kw)[0].cpu().numpy().astype(L) - true
+        err.append(float(np.sqrt((d * d).sum() / (true * true).sum())))
+    print(f"80 bits {(N, M)} rho {rho}: resident {err[0]:.2e}, steps {err[1]:.2e}", flush=True)
+    assert err[0] <= err[1] and err[0] <= 1e-16
 
 
 @pytest.mark.parametrize(("B", "N", "M"), [

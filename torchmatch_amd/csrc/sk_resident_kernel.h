@@ -83,6 +83,19 @@ template <> constexpr double kPHi<double> = 0x1p900;
 // float multipliers below this carry no rounding (their reciprocal overflows)
 constexpr float kCarryLo = 0x1p-120f;
 
+// (a - b) - d, d = a - b rounded (NaN or infinity where one of them is).
+__device__ __forceinline__ double diff_error(double a, double b, double d) {
+    const double bb = a - d;
+    return (a - (d + bb)) + (bb - b);
+}
+
+// damp * (lm - (ls + r)) with one rounding in place of three (float64 results).
+__device__ __forceinline__ double damped_potential(double damp, double lm, double ls, double r) {
+    const double t = ls + r, d = lm - t;
+    const double e = diff_error(lm, t, d) - diff_error(ls, -r, t);
+    return isfinite(e) ? fma(damp, d, damp * e) : damp * d;
+}
+
 // The log unit of each type: base 2 on the native v_exp_f32 for float costs,
 // natural with the library's exp / log for double costs.
 template <typename T> struct Unit;
@@ -104,8 +117,9 @@ template <> struct Unit<float> {
     static __device__ double of_nat(double x) { return x * kLog2eD; }
     static __device__ double to_nat(double x) { return x * kLn2D; }
     static __device__ double of_exp2(int e) { return (double)e; }
-    // P from its exponent, |error| about one ulp (NaN stays NaN)
-    static __device__ float build(double t) {
+    // P from its exponent K - l - c, |error| about one ulp (NaN stays NaN)
+    static __device__ float build(double k, double l, double c) {
+        double t = (k - l) - c;
         t = t < -300.0 ? -300.0 : t;
         const double ti = rint(t);
         return ldexpf(__builtin_amdgcn_exp2f((float)(t - ti)), (int)fmin(ti, 300.0));
@@ -125,7 +139,13 @@ template <> struct Unit<double> {
     static __device__ double of_nat(double x) { return x; }
     static __device__ double to_nat(double x) { return x; }
     static __device__ double of_exp2(int e) { return (double)e * kLn2D; }
-    static __device__ double build(double t) { return exp(t); }
+    // With what the two differences round off, which at |K| of 40 is up to 16 ulps
+    // of P in every step until P is built again.
+    static __device__ double build(double k, double l, double c) {
+        const double t = k - l, x = t - c;
+        const double p = exp(x), e = diff_error(k, l, t) + diff_error(t, c, x);
+        return isfinite(e) ? fma(p, e, p) : p;
+    }
 };
 
 __device__ __forceinline__ double shift_of(double m) { return isinf(m) ? 0.0 : m; }
@@ -1042,7 +1062,7 @@ sk_resident(const ResArgs A) {
                     const double l = S.rl[wr * RW + rs * r + h];
 #pragma unroll
                     for (int k = 0; k < TC; ++k) {
-                        v[r][k] = U::build((u.kval(v[r][k]) - l) - ck[k]);
+                        v[r][k] = U::build(u.kval(v[r][k]), l, ck[k]);
                         if (k % 4 == 3)
                             __builtin_amdgcn_sched_barrier(0);
                     }
@@ -1146,8 +1166,15 @@ sk_resident(const ResArgs A) {
                     if (!unbal) {
                         a_new = L.mu * U::recip(rsum);
                     } else {
-                        lu_new = damp * (L.lmu - (U::log_fast(rsum) + L.rl));
-                        a_new = U::exp_fast(lu_new + L.rl - kap);
+                        const double ls = U::log_fast(rsum);
+                        lu_new = damp * (L.lmu - (ls + L.rl));
+                        if constexpr (PW == 1) {
+                            a_new = U::exp_fast(lu_new + L.rl - kap);
+                        } else {  // (log_u is rounded to its own size, a need not be)
+                            a_new = U::exp_fast(damp * (L.lmu - ls) + ((1.0 - damp) * L.rl - kap));
+                            if (it + 1 == A.n_iter)
+                                lu_new = damped_potential(damp, L.lmu, ls, L.rl);
+                        }
                     }
                     const bool ok = L.dead ? rsum == 0.0
                                            : rsum >= kSumLo && rsum <= kSumHi && a_new <= kMulHi;
@@ -1355,9 +1382,14 @@ sk_resident(const ResArgs A) {
                         b_new[kc] = b;
                     } else {
                         const double c = cref[kc];
-                        const double lv =
-                            cdead[kc] ? cb[kc] : damp * (cnu[kc] - (U::log_fast(s) + c));
-                        b = U::exp_fast(lv + c - kap);
+                        const double ls = U::log_fast(s);
+                        double lv = cdead[kc] ? cb[kc] : damp * (cnu[kc] - (ls + c));
+                        if (PW > 1 && it + 1 == A.n_iter && !cdead[kc])
+                            lv = damped_potential(damp, cnu[kc], ls, c);
+                        if (PW == 1 || cdead[kc])
+                            b = U::exp_fast(lv + c - kap);
+                        else
+                            b = U::exp_fast(damp * (cnu[kc] - ls) + ((1.0 - damp) * c - kap));
                         b_new[kc] = lv;
                     }
                     const bool ok = cdead[kc] ? s == 0.0
