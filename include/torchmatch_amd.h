@@ -285,6 +285,10 @@ int tm_sinkhorn_iterate_f32(const float *cost, const uint8_t *keep, int64_t B, i
  * of 128 columns and more, a multiple of four), TM_SK_STEPS never. */
 enum { TM_SK_POTENTIALS = 0, TM_SK_PLAN = 1, TM_SK_STEPS = 2 };
 
+/* What one form needs (the queries without a form: the most any needs). */
+size_t tm_sinkhorn_workspace_bytes_form(int64_t B, int64_t N, int64_t M, int32_t form);
+size_t tm_sinkhorn_f64_workspace_bytes_form(int64_t B, int64_t N, int64_t M, int32_t form);
+
 /* The two halves with a form; give both the same. */
 int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *keep, const float *a,
                                  const float *b, int64_t B, int64_t N, int64_t M, float k_eps,

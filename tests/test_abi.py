@@ -42,6 +42,13 @@ def test_workspace_queries():
     assert lib.tm_jv_workspace_bytes_prefill(1024, 64, 64) == lib.tm_jv_workspace_bytes(1024, 64, 64)
     c3 = lib.tm_jv_workspace_bytes_prefill(64, 512, 768)
     assert lib.tm_jv_workspace_bytes(64, 512, 768) + 64 * 512 * 16 * 6 < c3 < 4 << 20
+    # plans (1), potentials (0), steps (2): a form pays for what it can run
+    form32 = [lib.tm_sinkhorn_workspace_bytes_form(2, 700, 300, f) for f in (1, 0, 2)]
+    assert form32[0] == lib.tm_sinkhorn_workspace_bytes(2, 700, 300) == form32[1] > form32[2]
+    form32 = [lib.tm_sinkhorn_workspace_bytes_form(2, 700, 90, f) for f in (1, 0, 2)]
+    assert form32[0] > form32[1] == form32[2]
+    form64 = [lib.tm_sinkhorn_f64_workspace_bytes_form(2, 700, 300, f) for f in (1, 0, 2)]
+    assert form64[0] == lib.tm_sinkhorn_f64_workspace_bytes(2, 700, 300) > form64[1] == form64[2]
     small = lib.tm_sinkhorn_workspace_bytes(2, 8, 8)
     big = lib.tm_sinkhorn_workspace_bytes(16, 2048, 2048)
     assert big > 16 * 2048 * 2048 * 4 > small

@@ -71,6 +71,12 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "tm_sinkhorn_workspace_bytes": (
         ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
     ),
+    "tm_sinkhorn_workspace_bytes_form": (
+        ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]
+    ),
+    "tm_sinkhorn_f64_workspace_bytes_form": (
+        ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]
+    ),
     "tm_sinkhorn_prepare_f32": (
         ctypes.c_int,
         [

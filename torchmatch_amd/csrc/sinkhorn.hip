@@ -239,7 +239,9 @@ void choose_fused(SinkhornLayout &L) {
     L.fz_interleave = f.W > 1;
 }
 
-SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
+// `form`: what runs resident in it (see resident_form) has room for that; the
+// statistics lie at the same place in every form.
+SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M, int32_t form) {
     SinkhornLayout L{};
     L.B = B;
     L.N = N;
@@ -264,7 +266,8 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
     choose_fused(L);
     // the variables that name a step form ask for that form
     L.res = SkResidentPlan{-1, 1, 0, 0, 1, 0};
-    if (getenv("TORCHMATCH_AMD_SINKHORN_FUSED") == nullptr &&
+    if ((form == TM_SK_PLAN || (form == TM_SK_POTENTIALS && L.fused != kFzNone)) &&
+        getenv("TORCHMATCH_AMD_SINKHORN_FUSED") == nullptr &&
         getenv("TORCHMATCH_AMD_SINKHORN_SHIFT_WINDOW") == nullptr)
         L.res = sk_resident_plan(B, N, M, false);
     const bool state64 = L.fused != kFzNone || L.res.cfg >= 0;
@@ -279,6 +282,8 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
     off = align_up(off + (size_t)(B * N), 256);
     L.off_infcol = off;
     off = align_up(off + (size_t)(B * M), 256);
+    L.off_stats = off;
+    off += 256;
     L.off_colpart = off;
     {
         int64_t parts = L.n_chunk > 1 ? L.n_chunk : 0;
@@ -310,8 +315,6 @@ SinkhornLayout make_layout(int64_t B, int64_t N, int64_t M) {
     L.off_lvw = off;
     if (L.fused)
         off = align_up(off + sizeof(float) * (size_t)(B * M), 256);
-    L.off_stats = off;
-    off += 256;
     L.off_xch = off;
     off = align_up(off + L.res.xch_bytes, 256);
     L.total = off;
@@ -346,20 +349,18 @@ __device__ __forceinline__ float k_of(float c, float e, double s2) {
     return s2 != 0.0 ? (float)((double)c * s2) : -c / e;
 }
 
-// `held` (may be null): the epsilon of K as it is in the workspace.  With
-// `unless_held` nothing is done where it is eps already; else it becomes eps.
+// `held`: the epsilon of K as it is in the workspace.  With `unless_held` nothing
+// is done where it is eps already; else it becomes eps.
 template <bool MASK>
 __global__ void __launch_bounds__(kMapBlock)
 sk_log_kernel(const float *__restrict__ C, const uint8_t *__restrict__ keep,
               float *__restrict__ K, int64_t n, float eps, double s2, int vec, float *held,
               int unless_held) {
-    if (held != nullptr) {
-        if (unless_held) {
-            if (*held == eps)
-                return;
-        } else if (blockIdx.x == 0 && threadIdx.x == 0) {
-            *held = eps;
-        }
+    if (unless_held) {
+        if (*held == eps)
+            return;
+    } else if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *held = eps;
     }
     const int64_t stride = (int64_t)gridDim.x * kMapBlock;
     const int64_t n4 = vec ? n / 4 : 0;
@@ -1650,10 +1651,15 @@ int grid_for(int64_t n, int block, int cap) {
 
 using namespace tmamd;
 
-extern "C" size_t tm_sinkhorn_workspace_bytes(int64_t B, int64_t N, int64_t M) {
+extern "C" size_t tm_sinkhorn_workspace_bytes_form(int64_t B, int64_t N, int64_t M,
+                                                   int32_t form) {
     if (B <= 0 || N <= 0 || M <= 0)
         return 256;
-    return make_layout(B, N, M).total;
+    return make_layout(B, N, M, form).total;
+}
+
+extern "C" size_t tm_sinkhorn_workspace_bytes(int64_t B, int64_t N, int64_t M) {
+    return tm_sinkhorn_workspace_bytes_form(B, N, M, TM_SK_PLAN);  // the largest form
 }
 
 namespace {
@@ -1903,7 +1909,7 @@ int launch_plan64(const SinkhornLayout &L, const FusedPtrs &P, const float *cost
     return TM_OK;
 }
 
-// Whether a call of this form runs resident (where the launch can).  Balanced
+// Which forms run resident (where the launch can; make_layout).  Balanced
 // potentials hold a neutral mode (a constant moved from log_u to log_v) that
 // every step's rounding feeds: the two-sweep step's natural-unit float32
 // potentials end up to 3e-4 of their norm from the float64 iteration's, the
@@ -1911,15 +1917,11 @@ int launch_plan64(const SinkhornLayout &L, const FusedPtrs &P, const float *cost
 // potentials gets those of the step its shape has always had, so the resident
 // solve takes such a call on the fused step's shapes only; plans, where
 // the constant cancels, differ by 1e-7 and take it everywhere.
-bool resident_form(const SinkhornLayout &L, int32_t form) {
-    return L.res.cfg >= 0 &&
-           (form == TM_SK_PLAN || (form == TM_SK_POTENTIALS && L.fused != kFzNone));
-}
+bool resident_form(const SinkhornLayout &L) { return L.res.cfg >= 0; }
 
 // Not under capture: a cooperative launch cannot be recorded.
-bool resident_ok(const SinkhornLayout &L, int32_t form, const void *workspace,
-                 hipStream_t stream) {
-    return resident_form(L, form) && ((uintptr_t)workspace % 16) == 0 && !stream_capturing(stream);
+bool resident_ok(const SinkhornLayout &L, const void *workspace, hipStream_t stream) {
+    return resident_form(L) && ((uintptr_t)workspace % 16) == 0 && !stream_capturing(stream);
 }
 
 } // namespace
@@ -1943,7 +1945,7 @@ extern "C" int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *ke
         return TM_OK;
     if (cost == nullptr || a == nullptr || b == nullptr)
         return TM_ERR_INVALID_ARGUMENT;
-    const SinkhornLayout L = make_layout(B, N, M);
+    const SinkhornLayout L = make_layout(B, N, M, form);
     if (workspace == nullptr || workspace_bytes < L.total)
         return TM_ERR_WORKSPACE;
     // prepare grid: y = row blocks of kPrepRows * groups rows (<= 65535)
@@ -1959,7 +1961,7 @@ extern "C" int tm_sinkhorn_prepare_form_f32(const float *cost, const uint8_t *ke
     uint8_t *inf_col = reinterpret_cast<uint8_t *>(ws + L.off_infcol);
     uint32_t *stats = reinterpret_cast<uint32_t *>(ws + L.off_stats);
 
-    if (resident_ok(L, form, workspace, stream))
+    if (resident_ok(L, workspace, stream))
         k_eps = 0.f;  // the resident solve reads the cost, not K
     int64_t n_flags = B * N > B * M ? B * N : B * M;
     n_flags = n_flags > kHeldWord ? n_flags : kHeldWord + 1;
@@ -2013,7 +2015,7 @@ extern "C" int tm_sinkhorn_read_stats(const void *workspace, int64_t B, int64_t 
         return TM_OK;
     if (workspace == nullptr)
         return TM_ERR_INVALID_ARGUMENT;
-    const SinkhornLayout L = make_layout(B, N, M);
+    const SinkhornLayout L = make_layout(B, N, M, TM_SK_STEPS);
     uint32_t words[2] = {0, 0};
     if (hipMemcpyAsync(words, static_cast<const char *>(workspace) + L.off_stats, sizeof(words),
                        hipMemcpyDeviceToHost, stream) != hipSuccess)
@@ -2068,7 +2070,7 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
     }
     if (cost == nullptr || log_u == nullptr || log_v == nullptr)
         return TM_ERR_INVALID_ARGUMENT;
-    const SinkhornLayout L = make_layout(B, N, M);
+    const SinkhornLayout L = make_layout(B, N, M, form);
     if (workspace == nullptr || workspace_bytes < L.total)
         return TM_ERR_WORKSPACE;
     if (!shape_supported(L))
@@ -2085,7 +2087,7 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
     const bool vec = (M % 4) == 0 && ((uintptr_t)log_v % 16) == 0;
     const bool fused = fused_ok(L, workspace);
 
-    if (resident_ok(L, form, workspace, stream)) {
+    if (resident_ok(L, workspace, stream)) {
         const FusedPtrs P = fused_ptrs(L, ws, log_u, log_v, 0);
         const SkResidentIo io{cost, keep, P.mu64, P.nu64, log_u, log_v, P.lu64, P.lv64,
                               ws + L.off_xch};
@@ -2100,8 +2102,8 @@ extern "C" int tm_sinkhorn_iterate_form_f32(const float *cost, const uint8_t *ke
     }
     // The preparation pass leaves K to this call when it expects it to run
     // resident (not under capture, say); which it did, the workspace knows.
-    float *held = L.res.cfg >= 0 ? reinterpret_cast<float *>(ws + L.off_stats) + kHeldWord : nullptr;
-    if (resident_form(L, form) && k_eps > 0.f) {
+    float *held = reinterpret_cast<float *>(ws + L.off_stats) + kHeldWord;
+    if (resident_form(L) && k_eps > 0.f) {
         const int rc = launch_log_kernel(cost, keep, K, nK, k_eps, fused, held, 1, stream);
         if (rc != TM_OK)
             return rc;

@@ -35,7 +35,8 @@ struct Layout64 {
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
-Layout64 layout64(int64_t B, int64_t N, int64_t M) {
+// Only TM_SK_PLAN runs resident (see tm_sinkhorn_form_f64).
+Layout64 layout64(int64_t B, int64_t N, int64_t M, int32_t form) {
     Layout64 L{};
     size_t off = 0;
     L.off_k = off;
@@ -48,7 +49,8 @@ Layout64 layout64(int64_t B, int64_t N, int64_t M) {
     off = align256(off + (size_t)(B * N));
     L.off_infcol = off;
     off = align256(off + (size_t)(B * M));
-    L.res = tmamd::sk_resident_plan(B, N, M, true);
+    L.res = form == TM_SK_PLAN ? tmamd::sk_resident_plan(B, N, M, true)
+                               : tmamd::SkResidentPlan{-1, 1, 0, 0, 1, 0};
     L.off_xch = off;
     off = align256(off + L.res.xch_bytes);
     L.total = off;
@@ -266,10 +268,15 @@ unsigned grid_for(int64_t n, int per, int64_t cap) {
 
 } // namespace
 
-extern "C" size_t tm_sinkhorn_f64_workspace_bytes(int64_t B, int64_t N, int64_t M) {
+extern "C" size_t tm_sinkhorn_f64_workspace_bytes_form(int64_t B, int64_t N, int64_t M,
+                                                       int32_t form) {
     if (B < 0 || N < 0 || M < 0)
         return 0;
-    return layout64(B, N, M).total;
+    return layout64(B, N, M, form).total;
+}
+
+extern "C" size_t tm_sinkhorn_f64_workspace_bytes(int64_t B, int64_t N, int64_t M) {
+    return tm_sinkhorn_f64_workspace_bytes_form(B, N, M, TM_SK_PLAN);  // the largest form
 }
 
 extern "C" int tm_sinkhorn_f64(const double *cost, const double *a, const double *b, int64_t B,
@@ -304,7 +311,7 @@ extern "C" int tm_sinkhorn_form_f64(const double *cost, const double *a, const d
         return TM_OK;  // no pair: the potentials keep their start value
     if (cost == nullptr || a == nullptr || b == nullptr)
         return TM_ERR_INVALID_ARGUMENT;
-    const Layout64 L = layout64(B, N, M);
+    const Layout64 L = layout64(B, N, M, form);
     if (workspace == nullptr || workspace_bytes < L.total)
         return TM_ERR_WORKSPACE;
     char *ws = static_cast<char *>(workspace);
@@ -326,7 +333,7 @@ extern "C" int tm_sinkhorn_form_f64(const double *cost, const double *a, const d
     // constant moved from log_u to log_v, 5e-14 of log_v's norm after 200 steps
     // against 4e-15 here), so a caller that reads them gets the steps below; in
     // plans the constant cancels.
-    if (form == TM_SK_PLAN && L.res.cfg >= 0 && !capturing && ((uintptr_t)workspace % 16) == 0) {
+    if (L.res.cfg >= 0 && !capturing && ((uintptr_t)workspace % 16) == 0) {
         const tmamd::SkResidentIo io{cost,  nullptr, log_mu,  log_nu,         log_u,
                                      log_v, nullptr, nullptr, ws + L.off_xch};
         const int rc = tmamd::sk_resident_launch(L.res, io, B, N, M, eps_sched, n_iter, rho, true,

@@ -195,7 +195,7 @@ sinkhorn_prepare_hip(const at::Tensor &cost, const c10::optional<at::Tensor> &ke
     TORCH_CHECK(b.dim() == 2 && b.size(0) == B && b.size(1) == M, "sinkhorn: b must be (B, M)");
     check_keep(cost, keep);
     const c10::DeviceGuard guard(cost.device());
-    const size_t ws_bytes = tm_sinkhorn_workspace_bytes(B, N, M);
+    const size_t ws_bytes = tm_sinkhorn_workspace_bytes_form(B, N, M, (int32_t)form);
     auto ws = at::empty({(int64_t)ws_bytes}, cost.options().dtype(at::kByte));
     const hipStream_t stream = current_stream(cost);
     if (read_stats)
@@ -271,7 +271,7 @@ sinkhorn_f64_hip(const at::Tensor &cost, const at::Tensor &a, const at::Tensor &
     auto log_v = at::empty({B, M}, cost.options());
     at::Tensor log_plan = write_plan ? at::empty({B, N, M}, cost.options())
                                      : at::empty({0}, cost.options());
-    const size_t ws_bytes = tm_sinkhorn_f64_workspace_bytes(B, N, M);
+    const size_t ws_bytes = tm_sinkhorn_f64_workspace_bytes_form(B, N, M, (int32_t)form);
     auto ws = at::empty({(int64_t)(ws_bytes > 0 ? ws_bytes : 1)}, cost.options().dtype(at::kByte));
     const int rc = tm_sinkhorn_form_f64(
         cost.data_ptr<double>(), a.data_ptr<double>(), b.data_ptr<double>(), B, N, M,
