@@ -89,8 +89,9 @@ SkResidentPlan sk_resident_plan(int64_t B, int64_t N, int64_t M, bool f64) {
                              mark_bytes(B);
         }
     }
-    // the streaming step: launches and merge, then the matrix at 7 TB/s, read
-    // twice by the two-sweep form (float64, odd and short rows)
+    // the streaming step: launches and merge, then 8.5 MB of the matrix a us
+    // (fitted up to the Infinity Cache's size, which serves part of it; HBM alone
+    // gives 6 to 7), read twice by the two-sweep form (float64, odd and short rows)
     const bool two = f64 || M % 4 != 0 || M < 128;
     const double mib = (f64 ? 8e-6 : 4e-6) * (double)(B * N * M);
     if (best.cfg >= 0 && best_t > 8.0 + mib / 8.5 * (two ? 2.0 : 1.0))

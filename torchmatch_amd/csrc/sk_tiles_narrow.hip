@@ -1,5 +1,6 @@
 // sk_tiles_narrow.hip -- resident Sinkhorn tiles of up to 256 columns (float32):
-// TC * TR entries per lane, at most 128 of its 256 VGPRs.
+// TC * TR entries per lane, at most 128 (of 512 VGPRs in four waves; in eight, of
+// 256, where the tiles of 128 spill: see sk_tiles_wide.hip).
 #include "sk_resident_kernel.h"
 
 namespace tmamd {

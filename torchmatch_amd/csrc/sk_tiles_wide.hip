@@ -1,4 +1,8 @@
-// sk_tiles_wide.hip -- resident Sinkhorn tiles of up to 4096 columns (float32).
+// sk_tiles_wide.hip -- resident Sinkhorn tiles of up to 4096 columns (float32): 24
+// to 128 entries per lane.  Four waves have 512 VGPRs a lane, eight have 256: there
+// the tiles of 128 entries spill about 120 and those of 96 up to 50 (hipcc's
+// report), in the building of P and around its calls; the products of a step read
+// none back, the rest of it some eight addresses.
 #include "sk_resident_kernel.h"
 
 namespace tmamd {
