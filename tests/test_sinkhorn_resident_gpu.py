@@ -257,6 +257,29 @@ def test_given_up(B, N, M, dtype, rho, device, monkeypatch):
         assert err <= (sk_parity.ELEM_BOUND if dtype == "float32" else 2e-13)
 
 
+@pytest.mark.parametrize("n", [2, 40, 600])
+def test_tiny_masses_that_drift(n, device):
+    """A row and a column of tiny mass that only have each other, in a problem
+    without a solution (row 0 alone cannot fill column 0), so that the potentials
+    drift by a factor a step: their multipliers become denormal while they are
+    all that some sums have."""
+    cost = torch.full((1, n, n), float("inf"))
+    k = n // 2  # k independent 2 x 2 problems
+    for i in range(k):
+        cost[0, 2 * i: 2 * i + 2, 2 * i: 2 * i + 2] = torch.tensor(
+            [[-19.32 + 0.01 * i, float("inf")], [-19.74, -19.30]])
+    a = torch.tensor([0.215, 7.85e-26]).repeat(k)[None] / k
+    b = torch.tensor([0.749, 2.51e-21]).repeat(k)[None] / k
+    ref = sk.log_sinkhorn_plan(cost, eps=2.0 ** -5, n_iter=50, a=a, b=b, dtype=torch.float64)[0]
+    got = solve(cost.to(device), reg=2.0 ** -5, n_iter=50, a=a.to(device), b=b.to(device))
+    sk_parity.logp_err(got, ref)  # the same entries finite
+    fin = torch.isfinite(ref)
+    d = (got.cpu().double() - ref).abs()[fin] / (1.0 + ref[fin].abs())
+    print(f"tiny masses {n}: {d.max().item():.2e}", flush=True)
+    # log plans down to -500, each rounded to 2^-24 of that, over potentials of 600
+    assert d.max().item() <= 1e-6
+
+
 @pytest.mark.skipif(np.finfo(np.longdouble).nmant < 63, reason="needs an 80-bit long double")
 @pytest.mark.parametrize(("N", "M", "eps", "n_iter", "rho"), [
     (300, 200, 0.05, 100, None), (64, 300, 0.1, 100, None), (300, 200, 0.05, 100, 1.0),

@@ -39,11 +39,12 @@
 // them before they are used.)  A step outside the window
 // (and the first) is done exactly from the cost, with the maximum taken out
 // of every sum, the reference's logsumexp, and P is rebuilt around the new
-// potentials.  Unbalanced multipliers have no lower bound (what underflows is
-// held as a potential, and contributes less than 2^-150 P to a sum), so a P
-// with an entry above 2^60 (both its row and its column carry less than 2^-60
-// of the mass) is refused there.  A row or column whose LSE is not finite keeps
-// its potential, as the reference's isfinite rule has it.  When epsilon changes, P is rebuilt
+// potentials.  Multipliers have no lower bound: a tiny one is denormal, off by
+// 2^-150, in the float32 copy that the products read, which is at most 2^-150 P of
+// a sum.  So a P with an entry above 2^60 is refused (its row and its column both
+// carry less than 2^-60 of the mass, or of the largest column's where there is a
+// kappa).  A row or column whose LSE is not finite keeps its potential, as the
+// reference's isfinite rule has it.  When epsilon changes, P is rebuilt
 // from the cost around the current potentials and the step goes on.
 //
 // Several workgroups per problem.  Each holds `rows` whole rows, so the row
@@ -77,9 +78,11 @@ namespace tmamd {
 namespace {
 
 constexpr double kSumLo = 0x1p-60, kSumHi = 0x1p60, kMulHi = 0x1p40;
-// unbalanced P above this is refused (kPHi<double>: doubles underflow 2^-1022)
+// P above this is refused (kPHi<double>: doubles underflow at 2^-1022); a balanced
+// entry of P is below 1 / mu of its row, so rows above kMassLo need no look
 template <typename T> constexpr T kPHi = (T)0x1p60;
 template <> constexpr double kPHi<double> = 0x1p900;
+constexpr double kMassLo = 0x1p-40;
 // float multipliers below this carry no rounding (their reciprocal overflows)
 constexpr float kCarryLo = 0x1p-120f;
 
@@ -1068,7 +1071,7 @@ sk_resident(const ResArgs A) {
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                if (unbal) {
+                if (unbal || ballot(has && W.mu < kMassLo) != 0) {
                     T top = (T)0;
 #pragma unroll
                     for (int r = 0; r < TR; ++r)
