@@ -338,6 +338,7 @@ template <typename F> struct Shared {
     float eb[F::KC * F::NT];
     uint8_t dead[F::KC * F::NT];
     int flag_row[2], flag_all[2], abort;
+    int look;  // P's largest entry is looked at (kPHi)
 };
 #define TM_LDS __attribute__((address_space(3)))
 template <typename F> using SharedP = TM_LDS Shared<F> *;
@@ -751,11 +752,16 @@ __device__ __noinline__ void start_problem(SharedP<F> S, const Job &J, Row &W, c
     using U = Unit<T>;
     const int t = (int)threadIdx.x;
     W = Row{-INFINITY, 0.0, 0.0, 0.0, 0.0, 0.f, false, false};
+    if (t == 0)
+        S->look = J.unbal;
+    __syncthreads();
     const int rho = lane_row(lane_id()), row = (t >> 6) / F::WC * F::RW + rho;
     if (rho < F::RW && row < J.nrow) {
         W.lmu = U::of_nat(lmu[row]);
         W.mu = U::expm(W.lmu);
         W.a = 1.0;
+        if (W.mu < kMassLo)
+            S->look = 1;
     }
     for (int j = t; j < F::CW; j += F::NT) {
         S->c[j] = j < J.M ? 0.0 : INFINITY;  // columns past M: P = 0, b = 0
@@ -1071,7 +1077,7 @@ sk_resident(const ResArgs A) {
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                if (unbal || ballot(has && W.mu < kMassLo) != 0) {
+                if (__builtin_expect(__builtin_amdgcn_readfirstlane(S.look) != 0, 0)) {
                     T top = (T)0;
 #pragma unroll
                     for (int r = 0; r < TR; ++r)
