@@ -35,11 +35,11 @@
 // an entry; a step is accepted only while every S_i and T_j lies in [2^-60,
 // 2^60] and every multiplier its sums use is at most 2^40, so that what is lost
 // is below 2^-150 2^40 2^17 (rows a problem may have) 2^60 = 2^-33 of a sum.
-// (The column multipliers of the first step may go to 2^60: P is rebuilt around
-// them before they are used.)  A step outside the window
-// (and the first) is done exactly from the cost, with the maximum taken out
-// of every sum, the reference's logsumexp, and P is rebuilt around the new
-// potentials.  Multipliers have no lower bound: a tiny one is denormal, off by
+// (The first step is a trial from P around the row maxima; its column multipliers
+// may go to 2^60, P is rebuilt around them before they are used.)  A step outside
+// the window is done exactly from the cost, with the maximum taken out of every
+// sum, the reference's logsumexp, and P is rebuilt around the new potentials.
+// Multipliers have no lower bound: a tiny one is denormal, off by
 // 2^-150, in the float32 copy that the products read, which is at most 2^-150 P of
 // a sum.  So a P with an entry above 2^60 is refused (its row and its column both
 // carry less than 2^-60 of the mass, or of the largest column's where there is a
